@@ -57,8 +57,10 @@ typedef void* orc_graph_t;  /* an instantiated hipGraphExec_t */
 typedef void* orc_event_t;  /* a hipEvent_t */
 
 /* ── runtime ─────────────────────────────────────────────────────────────── */
-/* Select `device`, create the default stream. Replaces nothing in the
- * reference (CPU-only); called once by the host before any other entry point. */
+/* Select `device`, create the default stream and allocate the workspace of
+ * the prefill GEMM (256 MB of device memory, shared by every call on the
+ * device and freed by orc_shutdown). Replaces nothing in the reference
+ * (CPU-only); called once by the host before any other entry point. */
 int orc_init(int device);
 int orc_shutdown(void);
 const char* orc_last_error(void);
@@ -112,12 +114,16 @@ int orc_embed(int type, const void* d_table, int n_in, int n_rows, const int32_t
 /* Y[t][j] = dot(X[t], dequant(W[j])) for t < n_tok, j < n_out, fp32
  * accumulation. n_tok = 1 is the decode GEMV (gemv_q / gemv_q_range,
  * core/gguf_parser.cpp:868-911); n_tok > 1 is the verify / prefill GEMM
- * (gemm_q, core/gguf_parser.cpp:919-997). The per-(token,row) reduction order
- * does not depend on n_tok, so the verify pass is bit-identical to n_tok
- * separate GEMVs. Supported types: Q4_0, Q8_0, Q4_K, Q6_K, and the dense
- * F32, F16 and BF16 (n_in a multiple of 32), which the reference runs through
- * its dequantize + ops::matmul fallback (core/model.cpp:370-381): fp32 FMA
- * on the exactly widened values, one kernel family at every token count. */
+ * (gemm_q, core/gguf_parser.cpp:919-997). Up to 23 tokens (every verify pass)
+ * the per-(token,row) reduction order does not depend on n_tok, so a verify
+ * pass is bit-identical to n_tok separate GEMVs (Q4_K / Q6_K: to other calls
+ * of two or more tokens). Calls of 24 tokens or more (prompt passes) of every
+ * type but F32 run the matrix-core prefill kernels: within fp32 rounding of
+ * the others, each token's row independent of the other tokens' values.
+ * Supported types: Q4_0, Q8_0, Q4_K, Q6_K, and the dense F32, F16 and BF16
+ * (n_in a multiple of 32), which the reference runs through its dequantize +
+ * ops::matmul fallback (core/model.cpp:370-381): fp32 sums over the exactly
+ * widened values. */
 int orc_gemm(int type, const void* d_w, int n_tok, int n_out, int n_in, const float* d_x, int ldx, float* d_y,
              int ldy, orc_stream_t stream);
 static inline int orc_gemv(int type, const void* d_w, int n_out, int n_in, const float* d_x, float* d_y,

@@ -5,10 +5,12 @@
 // them (RMSNorm, QKV bias, residual add, SwiGLU; core/model.cpp:366-473,
 // 565-643).
 //
-// Two kernel families. Q4_K and Q6_K matrices (a Q4_K_M target's) run on the
-// matrix cores (k_mmq, orc_mmq.hip); Q8_0 and Q4_0 on the vector ALUs (k_qmv,
-// below). Either way one matrix always uses one family and one reduction
-// order, so n-token results equal n decode results bit for bit.
+// Decode and verify calls (up to kPfSplitMin - 1 tokens) have two kernel
+// families: Q4_K and Q6_K matrices of two tokens or more run on the matrix
+// cores (k_mmq, orc_mmq.hip), everything else on the vector ALUs (k_qmv,
+// below), with one reduction order per family, so the tokens of a call are
+// independent bit for bit. Longer calls (prompt passes) of every type but F32
+// run on the matrix cores over activations split once (k_pf, orc_pf.hip).
 //
 // k_qmv design (n_tok = 1 is the decode GEMV):
 //  * Persistent 512-thread workgroups (one or two per CU). A workgroup stages
@@ -806,10 +808,10 @@ int gemm_device_init(int device) {
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && v > 0) g_n_cu = v;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && v > 0)
         g_lds_max = std::min<size_t>((size_t)v, 160 * 1024);
-    return ORC_OK;
+    return pf_init();
 }
 
-void gemm_device_release() {}
+void gemm_device_release() { pf_release(); }
 
 static int elems_per_unit(int type) { return type == ORC_Q6_K ? 64 : 32; }
 static int block_elems(int type) { return type == ORC_Q4_K || type == ORC_Q6_K || type == ORC_Q8_0_X8 ? 256 : 32; }
@@ -1015,10 +1017,16 @@ static int gemm_dispatch(QmvParams p, int type, hipStream_t s) {
     // the call's token count, never a chunk's, so chunking keeps results.
     const bool decode = p.n_tok == 1;
     if (decode && type == kMixK) return dispatch_mixed_decode(p, s);
+    if (pf_takes(type, p, s)) {
+        LaunchEvents ev;
+        if (g_prof_on) prof_arm(s, type, p.n_tok, gemm_bytes(p, p.n_tok), &ev.start, &ev.stop);
+        return pf_launch(type, p, s, ev);
+    }
     p.units = p.n_in / elems_per_unit(type);
     const bool mm = mmq_type(type) && !decode;
-    // a prefill pass (K-quant and Q8_0 calls of kPfMinTok tokens or more):
-    // every token in one launch on the matrix cores
+    // a prefill pass in a capture (K-quant and Q8_0 calls of kPfMinTok tokens
+    // or more; others went to pf_launch above): every token in one launch on
+    // the matrix cores, x staged by each workgroup
     if (!decode && (mm || type == ORC_Q8_0 || type == ORC_Q8_0_X8) && mmq_prefill(type, p)) {
         LaunchEvents ev;
         if (g_prof_on) prof_arm(s, type, p.n_tok, gemm_bytes(p, p.n_tok), &ev.start, &ev.stop);

@@ -52,10 +52,24 @@ int mmq_max_tokens(int type, const QmvParams& p);
 int mmq_launch(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev);
 // the same for launches whose wave ranges are staged in windows (orc_mmq_win.hip)
 int mmq_launch_windowed(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev);
-// Prefill launches (orc_mmq.hip): calls of at least kPfMinTok tokens on one
-// K-quant type run k_mmq_pf, all tokens in one launch.
+// Captured prefill launches (orc_mmq.hip): calls of at least kPfMinTok tokens
+// on one K-quant or Q8_0 type whose stream is being captured run k_mmq_pf, all
+// tokens in one launch, without a workspace.
 constexpr int kPfMinTok = 256;
 bool mmq_prefill(int type, const QmvParams& p);
 int mmq_prefill_launch(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev);
+
+// Prefill launches over split activations (orc_pf.hip): calls of at least
+// kPfSplitMin tokens, every type but F32, whose stream is not being captured.
+// The line: at 24 tokens the two launches and the split cost what the verify
+// kernels' 16-token block and its remainder do on the smallest K-quant matrix
+// (3072 x 3072 Q4_K: 21 us either way; at 20 tokens 21 against 18, at 32 21
+// against 27); every larger or vector-kernel matrix gains earlier (7B gate+up
+// Q6_K at 20 tokens 70 against 158 us). Verify passes stay below it.
+constexpr int kPfSplitMin = 24;
+int pf_init();
+void pf_release();
+bool pf_takes(int type, const QmvParams& p, hipStream_t s);
+int pf_launch(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev);
 
 }  // namespace orc

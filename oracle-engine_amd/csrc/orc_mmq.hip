@@ -13,10 +13,10 @@
 
 namespace orc {
 
-// ── prefill: 64 tokens per workgroup ────────────────────────────────────────
-// Calls of at least kPfMinTok tokens (the batched prefill of
-// Model::forward_prefill, core/model.cpp:510-674; verify passes are far
-// smaller) on Q4_K or Q6_K weights. One workgroup of eight waves per (block of
+// ── captured prefill: 64 tokens per workgroup ───────────────────────────────
+// Captured calls of at least kPfMinTok tokens on Q4_K, Q6_K or Q8_0 weights
+// (uncaptured ones run k_pf, orc_pf.hip, which needs the library's workspace).
+// One workgroup of eight waves per (block of
 // 128 rows, or of 128 SwiGLU gate / up row pairs, block of 64 tokens) walks
 // every unit of its rows once: each wave decodes its row tile's slice (the
 // same unit arithmetic as k_mmq: Q4_K scale folded into the codes, Q6_K

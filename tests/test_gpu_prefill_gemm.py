@@ -1,0 +1,223 @@
+"""The prefill GEMM over split activations (csrc/orc_pf.hip): calls of 24
+tokens and more on Q4_K, Q6_K, Q8_0 (GGUF and regrouped), Q4_0, F16 and BF16
+weights, against the float64 product of the oracle's dequantized rows.
+
+Bound, per (token, row), relative to sum |w x|: 2^-22 for the activations'
+split, and 2^-24 per rounding of the sum: at most 12 in a 32-value block (two
+MFMA steps of up to three pieces, two roundings each), 8 blocks per 256 values,
+at most 16 superblocks in a range, 16 ranges and the norm's 1/rms: 1.2e-7 *
+(2 + 12 + 8 + 16 + 16) / ... stays under 2e-6 even if every rounding had the
+same sign, at magnitudes that grow with the partial sum (half of the worst
+case on average). The wider tests of the same entry points (256 tokens and
+more) use the same 2e-6.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from conftest import rand_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(dev, oracle, qt, n_out, n_in, rng):
+    """(device buffer, weight type of the call, float64 values)"""
+    if qt == ol.BF16:
+        bits = (rng.normal(0, 0.05, n_out * n_in).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        return dev.upload(bits), qt, (bits.astype(np.uint32) << 16).view(np.float32).reshape(n_out, n_in).astype(np.float64)
+    gguf = ol.Q8_0 if qt == ol.Q8_0_X8 else qt
+    raw = rand_blocks(gguf, n_out * n_in, rng)
+    w = dev.upload(raw)
+    if qt == ol.Q8_0_X8:
+        dev.check(dev.L.orc_q8_0_regroup(w.ptr, n_out * n_in // 256, None))
+    return w, qt, oracle.dequant(gguf, raw, n_out * n_in).reshape(n_out, n_in).astype(np.float64)
+
+
+def _gemm(dev, qt, w, X, n_out, stream=None):
+    n_tok, n_in = X.shape
+    dx, dy = dev.upload(X), dev.alloc(n_tok * n_out * 4)
+    dev.sync()
+    dev.check(dev.L.orc_gemm(qt, w.ptr, n_tok, n_out, n_in, dx.ptr, n_in, dy.ptr, n_out, stream))
+    dev.sync()
+    return dy.read(np.float32).reshape(n_tok, n_out)
+
+
+def _check(got, X, W, tol=2e-6):
+    X = X.astype(np.float64)
+    err, scale = np.abs(got - X @ W.T), np.abs(X) @ np.abs(W).T
+    assert np.all(err <= tol * scale + 1e-30), float(np.max(err / (scale + 1e-300)))
+
+
+# tile edges: 32 / 64 / 128 tokens, 32 and 128 rows; K of less than a
+# superblock, of whole and of partial ones (896 and 1120 values: Q8_0, Q4_0
+# and dense rows), and long enough to be split into several ranges
+CASES = [(ol.Q4_K, 24, 31, 256), (ol.Q4_K, 33, 130, 2304), (ol.Q6_K, 32, 33, 256), (ol.Q6_K, 65, 127, 4352),
+         (ol.Q8_0, 25, 129, 32), (ol.Q8_0, 64, 64, 896), (ol.Q8_0, 129, 97, 1120), (ol.Q8_0_X8, 128, 32, 2048),
+         (ol.Q4_0, 31, 40, 1120), (ol.Q4_0, 193, 128, 96), (ol.F16, 63, 257, 4352), (ol.F16, 127, 16, 160),
+         (ol.BF16, 40, 96, 4352), (ol.BF16, 130, 161, 96), (ol.Q6_K, 130, 17000, 256), (ol.F16, 300, 17000, 64)]
+
+
+@pytest.mark.parametrize("qt,nt,n_out,n_in", CASES)
+def test_against_float64(dev, oracle, qt, nt, n_out, n_in):
+    print(f"[gpu] pf gemm type={qt} nt={nt} {n_out}x{n_in}", flush=True)
+    rng = np.random.default_rng(nt + n_out)
+    w, ty, W = _weights(dev, oracle, qt, n_out, n_in, rng)
+    X = (rng.normal(0, 1, (nt, n_in)) * 10.0 ** rng.integers(-6, 6, (nt, 1))).astype(np.float32)
+    X[nt // 2] = 0.0
+    got = _gemm(dev, ty, w, X, n_out)
+    _check(got, X, W)
+    assert not got[nt // 2].any()
+    # a token's row does not depend on the other tokens of a call of this size
+    Y = rng.normal(0, 1, X.shape).astype(np.float32)
+    Y[3] = X[3]
+    assert np.array_equal(_gemm(dev, ty, w, Y, n_out)[3], got[3])
+
+
+@pytest.mark.parametrize("qt,nt,n_in", [(ol.Q4_K, 50, 512), (ol.Q8_0, 40, 864), (ol.F16, 140, 4352)])
+def test_epilogues(dev, oracle, qt, nt, n_in):
+    """RMSNorm prologue with bias into three segments, SwiGLU pairs (rows not a
+    multiple of 16) and residual accumulation, in float64."""
+    import orc
+
+    print(f"[gpu] pf epilogues type={qt} nt={nt} n_in={n_in}", flush=True)
+    rng = np.random.default_rng(7 * nt)
+    rows = (45, 33, 50)
+    ws = [_weights(dev, oracle, qt, r, n_in, rng) for r in rows]
+    X = rng.normal(0, 3, (nt, n_in)).astype(np.float32)
+    g = rng.uniform(0.5, 1.5, n_in).astype(np.float32)
+    dx, dg = dev.upload(X), dev.upload(g)
+    Xd = X.astype(np.float64)
+    Xn = Xd / np.sqrt((Xd ** 2).mean(1, keepdims=True) + 1e-5) * g
+    dot = [Xn @ W.T for _, _, W in ws]
+    scale = [np.abs(Xn) @ np.abs(W).T for _, _, W in ws]
+    ld = sum(rows)
+    bias = rng.normal(0, 1, rows[1]).astype(np.float32)
+    db, dy = dev.upload(bias), dev.alloc(nt * ld * 4)
+    offs = np.cumsum((0,) + rows)
+    segs = (orc.Seg * 3)(*[orc.Seg(w[0].ptr, r, dy.ptr + int(o) * 4, db.ptr if i == 1 else None)
+                           for i, (w, r, o) in enumerate(zip(ws, rows, offs))])
+    dev.check(dev.L.orc_gemm_fused(qt, segs, 3, nt, n_in, dx.ptr, n_in, ld, dg.ptr, C.c_float(1e-5), orc.EPI_STORE,
+                                   None))
+    got = dy.read(np.float32).reshape(nt, ld)
+    for i, r in enumerate(rows):
+        want = dot[i] + (bias if i == 1 else 0)
+        assert np.all(np.abs(got[:, offs[i]:offs[i + 1]] - want) <= 2e-6 * scale[i] + 3e-7 * np.abs(want)), i
+    # SwiGLU over the first rows of two segments
+    ff = 33
+    segs = (orc.Seg * 2)(orc.Seg(ws[0][0].ptr, ff, dy.ptr, None), orc.Seg(ws[1][0].ptr, ff, dy.ptr, None))
+    dev.check(dev.L.orc_gemm_fused(qt, segs, 2, nt, n_in, dx.ptr, n_in, ff, dg.ptr, C.c_float(1e-5), orc.EPI_SWIGLU,
+                                   None))
+    got = dy.read(np.float32, nt * ff).reshape(nt, ff)
+    gt, up = dot[0][:, :ff], dot[1]
+    want = gt / (1 + np.exp(-gt)) * up
+    tol = 3e-6 * (scale[0][:, :ff] * np.abs(up) + scale[1] * np.abs(gt)) + 1e-6 * np.abs(want) + 1e-30
+    assert np.all(np.abs(got - want) <= tol)  # |silu'| <= 1.1
+    res = rng.normal(0, 1, (nt, rows[2])).astype(np.float32)
+    dr = dev.upload(res)
+    segs = (orc.Seg * 1)(orc.Seg(ws[2][0].ptr, rows[2], dr.ptr, None))
+    dev.check(dev.L.orc_gemm_fused(qt, segs, 1, nt, n_in, dx.ptr, n_in, rows[2], None, C.c_float(0), orc.EPI_ACCUM,
+                                   None))
+    W = ws[2][2]
+    want = res + Xd @ W.T
+    assert np.all(np.abs(dr.read(np.float32).reshape(nt, -1) - want) <=
+                  2e-6 * (np.abs(Xd) @ np.abs(W).T) + 1.2e-7 * np.abs(want))
+
+
+def test_mixed_segments(dev, oracle):
+    """Q4_K and Q6_K segments of one call (a Q4_K_M layer's Q|K|V) share one split."""
+    import orc
+
+    rng = np.random.default_rng(5)
+    n_in, rows, types, nt = 1024, (96, 32, 64), (ol.Q4_K, ol.Q6_K, ol.Q6_K), 70
+    ws = [_weights(dev, oracle, t, r, n_in, rng) for t, r in zip(types, rows)]
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    dx, dy = dev.upload(X), dev.alloc(nt * sum(rows) * 4)
+    offs = np.cumsum((0,) + rows)
+    segs = (orc.Seg * 3)(*[orc.Seg(w[0].ptr, r, dy.ptr + int(o) * 4, None) for w, r, o in zip(ws, rows, offs)])
+    ty = (C.c_int32 * 3)(*types)
+    dev.check(dev.L.orc_gemm_fused_mixed(ty, segs, 3, nt, n_in, dx.ptr, n_in, sum(rows), None, C.c_float(0),
+                                         orc.EPI_STORE, None))
+    got = dy.read(np.float32).reshape(nt, -1)
+    for i in range(3):
+        _check(got[:, offs[i]:offs[i + 1]], X, ws[i][2])
+
+
+@pytest.mark.parametrize("qt", [ol.Q8_0, ol.F16, ol.BF16])
+def test_infinities_and_nan_stay_in_their_token(dev, oracle, qt):
+    """An infinite activation gives the infinity (or NaN) of the fp32 product
+    in its own row, whatever else the row holds; other tokens are untouched."""
+    rng = np.random.default_rng(3)
+    n_in, n_out, nt = 512, 40, 30
+    w, ty, W = _weights(dev, oracle, qt, n_out, n_in, rng)
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    clean = _gemm(dev, ty, w, X, n_out)
+    X[4, 100] = np.inf
+    X[4, 101] = 1e6  # finite neighbours keep their scale
+    X[9, 7] = np.nan
+    got = _gemm(dev, ty, w, X, n_out)
+    W32 = W[:, 100]
+    assert np.array_equal(got[4][W32 > 0], np.full((W32 > 0).sum(), np.inf, np.float32))
+    assert np.array_equal(got[4][W32 < 0], np.full((W32 < 0).sum(), -np.inf, np.float32))
+    assert np.isnan(got[9]).all()
+    keep = [t for t in range(nt) if t not in (4, 9)]
+    assert np.array_equal(got[keep], clean[keep])
+
+
+def test_streams_take_the_workspace_in_turn(dev, oracle):
+    """Calls interleaved on two streams, without waiting in between, equal
+    the same calls one after another bit for bit."""
+    rng = np.random.default_rng(11)
+    n_in, n_out, nt = 2048, 512, 200
+    w, ty, W = _weights(dev, oracle, ol.Q6_K, n_out, n_in, rng)
+    Xs = [rng.normal(0, 1, (nt, n_in)).astype(np.float32) for _ in range(6)]
+    want = [_gemm(dev, ty, w, X, n_out) for X in Xs]
+    dxs, dys = [dev.upload(X) for X in Xs], [dev.alloc(nt * n_out * 4) for _ in Xs]
+    streams = [C.c_void_p() for _ in range(2)]
+    for s in streams:
+        dev.check(dev.L.orc_stream_create(C.byref(s)))
+    dev.sync()
+    for i, (dx, dy) in enumerate(zip(dxs, dys)):
+        dev.check(dev.L.orc_gemm(ty, w.ptr, nt, n_out, n_in, dx.ptr, n_in, dy.ptr, n_out, streams[i % 2]))
+    dev.sync()
+    for dy, e in zip(dys, want):
+        assert np.array_equal(dy.read(np.float32).reshape(nt, n_out), e)
+    for s in streams:
+        dev.check(dev.L.orc_stream_destroy(s))
+
+
+def test_captured_calls_do_not_use_the_workspace(dev, oracle):
+    """A captured call (it keeps the kernels that stage x themselves) replays
+    to the same values while other calls use the workspace in between."""
+    rng = np.random.default_rng(12)
+    n_in, n_out, nt = 1024, 256, 48
+    w, ty, W = _weights(dev, oracle, ol.Q4_K, n_out, n_in, rng)
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    dx, dy = dev.upload(X), dev.alloc(nt * n_out * 4)
+    s, graph = C.c_void_p(), C.c_void_p()
+    dev.check(dev.L.orc_stream_create(C.byref(s)))
+    dev.check(dev.L.orc_graph_begin(s))
+    dev.check(dev.L.orc_gemm(ty, w.ptr, nt, n_out, n_in, dx.ptr, n_in, dy.ptr, n_out, s))
+    dev.check(dev.L.orc_graph_end(s, C.byref(graph)))
+    outs = []
+    for _ in range(3):
+        dev.check(dev.L.orc_graph_launch(graph, s))
+        _check(_gemm(dev, ty, w, X[::-1].copy(), n_out), X[::-1], W)  # eager work beside the replay
+        dev.sync()
+        outs.append(dy.read(np.float32).reshape(nt, n_out))
+        _check(outs[-1], X, W)
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+    dev.check(dev.L.orc_graph_destroy(graph))
+    dev.check(dev.L.orc_stream_destroy(s))
+
+
+def test_token_chunks(dev, oracle):
+    """More tokens than the workspace holds at once go in chunks."""
+    rng = np.random.default_rng(13)
+    n_in, n_out, nt = 18944, 20, 3600
+    w, ty, W = _weights(dev, oracle, ol.Q6_K, n_out, n_in, rng)
+    X = rng.standard_normal((nt, n_in), np.float32)
+    got = _gemm(dev, ty, w, X, n_out)
+    pick = np.r_[0:40, 3400:3600]  # both sides of the chunk boundary
+    _check(got[pick], X[pick], W)
