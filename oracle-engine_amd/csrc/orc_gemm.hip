@@ -1018,9 +1018,16 @@ static int gemm_dispatch(QmvParams p, int type, hipStream_t s) {
     const bool decode = p.n_tok == 1;
     if (decode && type == kMixK) return dispatch_mixed_decode(p, s);
     if (pf_takes(type, p, s)) {
-        LaunchEvents ev;
-        if (g_prof_on) prof_arm(s, type, p.n_tok, gemm_bytes(p, p.n_tok), &ev.start, &ev.stop);
-        return pf_launch(type, p, s, ev);
+        uint8_t* work = nullptr;
+        int rc = pf_ws_begin(s, &work);
+        if (!rc) {
+            LaunchEvents ev;
+            if (g_prof_on) prof_arm(s, type, p.n_tok, gemm_bytes(p, p.n_tok), &ev.start, &ev.stop);
+            rc = pf_launch(type, p, s, ev, work);
+            const int re = pf_ws_end(s);
+            return rc ? rc : re;
+        }
+        if (rc != kPfBusy) return rc;
     }
     p.units = p.n_in / elems_per_unit(type);
     const bool mm = mmq_type(type) && !decode;

@@ -6,6 +6,8 @@
 // of Model::forward (core/model.cpp:401-435) and Model::forward_prefill
 // (core/model.cpp:595-626), and the acceptance step of the batched spec loop
 // (benchmark/bench_engine.cpp:337-355).
+#include "orc_attn_pf.hpp"
+#include "orc_gemm.hpp"
 #include "orc_internal.hpp"
 #include <hip/hip_ext.h>
 
@@ -1667,7 +1669,16 @@ extern "C" int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_
         bytes += 8.0 * n_kv * head_dim * (pos_off + std::min(n_tok, t0 + kPaTok));
     bytes += 4.0 * n_tok * ((double)(n_heads + 2 * n_kv) * head_dim + (double)n_heads * head_dim);
     LaunchEv ev;
+    uint8_t* work = nullptr;
+    int rc = pf_ws_takes(st, fa_bytes(head_dim, n_kv, pos_off + n_tok)) ? pf_ws_begin(st, &work) : kPfBusy;
+    if (rc && rc != kPfBusy) return rc;
     const bool tm = prof_arm(st, kProfAttnPf, n_tok, bytes, &ev.a, &ev.b);
+    if (!rc) {
+        const FaArgs a{d_qkv, ldqkv, n_tok, n_heads, n_kv, pos_off, (const float2*)d_rope, d_kc, d_vc, ctx, d_out, ldo, st};
+        rc = fa_launch(head_dim, a, work, tm ? ev.a : nullptr, tm ? ev.b : nullptr);
+        const int re = pf_ws_end(st);
+        return rc ? rc : re;
+    }
     if (head_dim == 64) {
         const size_t lds = pa_lds_bytes<64>(R);
         if (lds > 160 * 1024) return set_error(ORC_E_UNSUPPORTED, "attn_prefill: LDS");

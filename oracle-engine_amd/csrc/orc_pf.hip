@@ -686,38 +686,66 @@ __global__ __launch_bounds__(64 * RW) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
 }
 
-// Sum of the ranges' partial results in range order, then the epilogue: one
-// thread per output value. Bound by memory (a few MB).
+// Sum of the ranges' partial results in range order, then the epilogue: four
+// output values per thread, the loads of four ranges in flight. Bound by
+// memory (a few MB).
+constexpr int kSumV = 4;
 __global__ __launch_bounds__(256) void k_pf_sum(QmvParams p, PfWork wk, const float* part, int nz) {
-    const int j = blockIdx.x * 256 + threadIdx.x, tok = blockIdx.y;
+    const int tok = blockIdx.y, j0 = blockIdx.x * (256 * kSumV) + threadIdx.x;
     const bool swiglu = p.epi == ORC_EPI_SWIGLU;
-    if (j >= (swiglu ? p.rows[0] : p.n_rows)) return;
-    const float* s = part + (size_t)tok * p.n_rows + j;
+    const int rows = swiglu ? p.rows[0] : p.n_rows;
     const size_t zs = (size_t)p.n_tok * p.n_rows;
-    float v = 0.f, u = 0.f;
-    for (int z = 0; z < nz; ++z) {
-        v += s[z * zs];
-        if (swiglu) u += s[z * zs + p.rows[0]];
-    }
+    auto sum = [&](const float* s, float (&v)[kSumV]) {
+#pragma unroll
+        for (int k = 0; k < kSumV; ++k) v[k] = 0.f;
+        for (int z0 = 0; z0 < nz; z0 += 4) {
+            float t[4][kSumV];
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+#pragma unroll
+                for (int k = 0; k < kSumV; ++k)
+                    t[z][k] = *(gfp)(s + min(z0 + z, nz - 1) * zs + min(j0 + 256 * k, rows - 1));
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+#pragma unroll
+                for (int k = 0; k < kSumV; ++k)
+                    if (z0 + z < nz) v[k] += t[z][k];
+        }
+    };
+    float v[kSumV], u[kSumV];
+    const float* s = part + (size_t)tok * p.n_rows;
+    sum(s, v);
+    if (swiglu) sum(s + rows, u);
     const float inv = p.norm_w ? pf_inv_rms(wk, tok >> 5, tok & 31, p.n_in, p.eps) : 1.f;
-    int jj;
-    const int sg = seg_of(j, p.n_seg, p.rows[0], p.rows[1], jj);
-    float* y = swiglu ? p.y[0] + j : pick3(sg, p.y[0], p.y[1], p.y[2]) + jj;
-    const float* bb = swiglu ? nullptr : pick3(sg, p.bias[0], p.bias[1], p.bias[2]);
-    pf_write(p, y + (size_t)tok * p.ldy, v * inv, u * inv, bb ? bb[jj] : 0.f);
+#pragma unroll
+    for (int k = 0; k < kSumV; ++k) {
+        const int j = j0 + 256 * k;
+        if (j >= rows) continue;
+        int jj;
+        const int sg = seg_of(j, p.n_seg, p.rows[0], p.rows[1], jj);
+        float* y = swiglu ? p.y[0] + j : pick3(sg, p.y[0], p.y[1], p.y[2]) + jj;
+        const float* bb = swiglu ? nullptr : pick3(sg, p.bias[0], p.bias[1], p.bias[2]);
+        pf_write(p, y + (size_t)tok * p.ldy, v[k] * inv, swiglu ? u[k] * inv : 0.f, bb ? bb[jj] : 0.f);
+    }
 }
 
 // ── workspace ────────────────────────────────────────────────────────────────
 // One per device, allocated by orc_init and freed by orc_shutdown (or when
 // orc_init selects another device). A call holds the lock while it enqueues
-// its launches, waits (on its stream) for the event of the call before and
-// records its own, so calls of any streams and threads take the workspace in
-// turn. kPfWorkBytes holds 1024 tokens of 18944 values with their side arrays
-// (83 MB); calls that need more go in token chunks.
-constexpr size_t kPfWorkBytes = (size_t)256 << 20;
+// its launches, and its stream first waits for the last use on any other
+// stream, so calls of any streams and threads take the workspace in turn.
+// Uses that follow each other on one of the library's own streams need no
+// event: the one a change of stream waits for is recorded then (or when the
+// stream is destroyed). An event after every use costs 4.4 us of GPU time
+// between two calls (3B blocks at 127 tokens: 22 of 222 us a layer). A stream
+// the library did not create may be destroyed behind its back, so its uses
+// are followed by an event at once.
+// GEMM calls that need more than kPfWorkBytes go in token chunks.
 static std::mutex g_pf_mu;
 static uint8_t* g_pf_buf = nullptr;
 static hipEvent_t g_pf_ev = nullptr;
+static bool g_pf_ev_set = false;         // g_pf_ev follows the last use
+static hipStream_t g_pf_last = nullptr;  // or the last use is on this stream of the library
 
 void pf_release() {
     std::lock_guard<std::mutex> lk(g_pf_mu);
@@ -725,14 +753,59 @@ void pf_release() {
     if (g_pf_ev) (void)hipEventDestroy(g_pf_ev);
     g_pf_buf = nullptr;
     g_pf_ev = nullptr;
+    g_pf_ev_set = false;
+    g_pf_last = nullptr;
 }
 
 int pf_init() {
     pf_release();
     std::lock_guard<std::mutex> lk(g_pf_mu);
     ORC_HIP_CHECK(hipMalloc((void**)&g_pf_buf, kPfWorkBytes));
-    ORC_HIP_CHECK(hipEventCreateWithFlags(&g_pf_ev, hipEventDisableTiming));
+    ORC_HIP_CHECK(hipEventCreateWithFlags(&g_pf_ev, hipEventDisableTiming | hipEventDisableSystemFence));
     return ORC_OK;
+}
+
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
+bool pf_ws_takes(hipStream_t s, size_t bytes) { return g_pf_buf && bytes <= kPfWorkBytes && !capturing(s); }
+
+int pf_ws_begin(hipStream_t s, uint8_t** buf) {
+    std::unique_lock<std::mutex> lk(g_pf_mu);
+    if (!g_pf_buf) return set_error(ORC_E_NOINIT, "orc_init not called");
+    if (g_pf_last != s) {
+        if (g_pf_last) {
+            if (capturing(g_pf_last)) return kPfBusy;  // it cannot record an event now
+            ORC_HIP_CHECK(hipEventRecord(g_pf_ev, g_pf_last));
+            g_pf_last = nullptr;
+            g_pf_ev_set = true;
+        }
+        if (g_pf_ev_set) ORC_HIP_CHECK(hipStreamWaitEvent(s, g_pf_ev, 0));
+    }
+    *buf = g_pf_buf;
+    lk.release();  // held until pf_ws_end
+    return ORC_OK;
+}
+
+int pf_ws_end(hipStream_t s) {
+    std::unique_lock<std::mutex> lk(g_pf_mu, std::adopt_lock);
+    if (library_stream(s)) {
+        g_pf_last = s;
+        return ORC_OK;
+    }
+    g_pf_last = nullptr;
+    g_pf_ev_set = true;
+    ORC_HIP_CHECK(hipEventRecord(g_pf_ev, s));
+    return ORC_OK;
+}
+
+void pf_ws_forget(hipStream_t s) {
+    std::lock_guard<std::mutex> lk(g_pf_mu);
+    if (g_pf_last != s) return;
+    g_pf_last = nullptr;
+    g_pf_ev_set = hipEventRecord(g_pf_ev, s) == hipSuccess;
 }
 
 struct PfType {
@@ -781,7 +854,7 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
         hipLaunchKernelGGL((k_pf<QT, RW, TT>), grid, dim3(64 * RW), lds, s, p, w, pt);
     ORC_LAUNCH_CHECK();
     if (!pt) return ORC_OK;
-    const dim3 g2((rows + 255) / 256, p.n_tok);
+    const dim3 g2((rows + 256 * kSumV - 1) / (256 * kSumV), p.n_tok);
     if (stop) hipExtLaunchKernelGGL(k_pf_sum, g2, dim3(256), 0, s, nullptr, stop, 0, p, w, (const float*)part, nz);
     else hipLaunchKernelGGL(k_pf_sum, g2, dim3(256), 0, s, p, w, (const float*)part, nz);
     ORC_LAUNCH_CHECK();
@@ -794,11 +867,12 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
 //  * 128 rows x 32 tokens for at most 32 tokens (7B gate+up Q6_K 75 against
 //    90 with 64-token tiles);
 //  * 128 x 128 once such tiles are two per CU (7B gate+up, 1023 tokens: 891
-//    against 1024 with 128 x 64; 2048-wide Q4_0 216 against 270), not for
-//    BF16, whose three pieces per value leave one such workgroup per CU (332
-//    against 262);
+//    against 1024 with 128 x 64; 2048-wide Q4_0 216 against 270) and K is at
+//    least eight superblocks (0.5B gate+up, n_in 896: 110 against 87), not
+//    for BF16, whose three pieces per value leave one such workgroup per CU
+//    (332 against 262);
 //  * 128 x 64 otherwise (3072 x 3072 Q4_K, 1023 tokens: 84 against 107).
-//  * K is split while the tiles leave CUs idle: about 640 workgroups, ranges
+//  * K is split while the tiles leave CUs idle: up to 768 workgroups, ranges
 //    of at least two superblocks (three above 128 tokens, where the partial
 //    sums weigh more): 3584 x 18944 at 127 tokens 364 in one range, 106 in
 //    eight; 3584 x 3584 83 -> 38; F16 2048 x 8192 142 -> 34. F16 and BF16
@@ -814,10 +888,10 @@ static PfPlan pf_plan(int type, const QmvParams& p, int supers) {
     auto wgs = [&](int bt) { return (long)((rows + 127) / 128) * ((p.n_tok + bt - 1) / bt); };
     PfPlan r{1, 1};
     if (p.n_tok <= 32) r.shape = 2;
-    else if (type != ORC_BF16 && p.n_tok > 64 && wgs(128) >= 2 * g_n_cu) r.shape = 0;
-    const long w = wgs(r.shape == 0 ? 128 : r.shape == 1 ? 64 : 32), want = 5 * g_n_cu / 2;
+    else if (type != ORC_BF16 && p.n_tok > 64 && supers >= 8 && wgs(128) >= 2 * g_n_cu) r.shape = 0;
+    const long w = wgs(r.shape == 0 ? 128 : r.shape == 1 ? 64 : 32), want = 3 * g_n_cu;
     const int most = std::min(16, std::max(1, (supers + 1) / (p.n_tok <= 128 ? 2 : 3)));
-    r.nz = (int)std::min<long>(most, (want + w - 1) / w);
+    r.nz = (int)std::max<long>(1, std::min<long>(most, want / w));
     if (dense) r.nz = std::max(r.nz, (supers + 15) / 16);
     return r;
 }
@@ -844,27 +918,22 @@ static int pf_split(const PfType& t, const PfSplit& sp, int ng, hipStream_t s, h
 }
 
 bool pf_takes(int type, const QmvParams& p, hipStream_t s) {
-    if (p.n_tok < kPfSplitMin || !g_pf_buf || p.n_in % 32) return false;
+    if (p.n_tok < kPfSplitMin || p.n_in % 32) return false;
     PfType t;
     if (type == kMixK) t = {2, true, true};
     else if (!pf_type(type, t)) return false;
     if (p.epi == ORC_EPI_SWIGLU && p.n_seg != 2) return false;
     PfWork w;
-    if (pf_layout(t, p.n_in, 4, nullptr, w) > kPfWorkBytes) return false;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    return pf_ws_takes(s, pf_layout(t, p.n_in, 4, nullptr, w));
 }
 
-int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& ev) {
+int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& ev, uint8_t* buf) {
     PfType t;
     if (type == kMixK) t = {2, true, true};  // Q4_K and Q6_K segments share one split
     else if (!pf_type(type, t)) return set_error(ORC_E_INVALID, "gemm: not a prefill launch");
     PfWork w;
     const size_t per4 = pf_layout(t, p0.n_in, 4, nullptr, w);  // 128 tokens
     const int chunk = (int)std::min<size_t>(kPfWorkBytes / per4, 1 << 20) * 128;
-    std::lock_guard<std::mutex> lk(g_pf_mu);
-    if (!g_pf_buf) return set_error(ORC_E_NOINIT, "orc_init not called");
-    ORC_HIP_CHECK(hipStreamWaitEvent(s, g_pf_ev, 0));
     int rc = ORC_OK;
     for (int t0 = 0; t0 < p0.n_tok && !rc; t0 += chunk) {
         QmvParams p = p0;
@@ -872,7 +941,7 @@ int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& 
         p.x = p0.x + (size_t)t0 * p0.ldx;
         for (int i = 0; i < 3; ++i) p.y[i] = p0.y[i] ? p0.y[i] + (size_t)t0 * p0.ldy : nullptr;
         const int ng = p.n_tok <= 64 ? 2 : (p.n_tok + 127) / 128 * 4;
-        const size_t used = pf_layout(t, p.n_in, ng, g_pf_buf, w);
+        const size_t used = pf_layout(t, p.n_in, ng, buf, w);
         PfSplit sp{w, p.x, p.norm_w, p.ldx, p.n_tok, p.n_in};
         if ((rc = pf_split(t, sp, ng, s, t0 == 0 ? ev.start : nullptr))) break;
         // one launch per run of segments of one type
@@ -893,7 +962,7 @@ int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& 
             q.row_bytes = p.seg_rb[i0];
             const hipEvent_t stop = i1 == p.n_seg && t0 + chunk >= p0.n_tok ? ev.stop : nullptr;
             PfPlan r = pf_plan(p.seg_type[i0], q, w.supers);
-            float* const part = (float*)(g_pf_buf + used);  // partial sums behind the split activations
+            float* const part = (float*)(buf + used);  // partial sums behind the split activations
             r.nz = (int)std::min<size_t>(r.nz, std::max<size_t>(1, (kPfWorkBytes - used) / ((size_t)p.n_tok * q.n_rows * 4)));
             switch (p.seg_type[i0]) {
                 case ORC_Q4_K: rc = pf_run<ORC_Q4_K>(q, w, r, part, s, stop); break;
@@ -908,11 +977,7 @@ int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& 
             i0 = i1;
         }
     }
-    // recorded whatever was enqueued: the next call waits for it
-    const hipError_t e = hipEventRecord(g_pf_ev, s);
-    if (rc) return rc;
-    if (e != hipSuccess) return set_error(ORC_E_HIP, std::string("hipEventRecord: ") + hipGetErrorString(e));
-    return ORC_OK;
+    return rc;
 }
 
 }  // namespace orc

@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <unordered_set>
 
 namespace orc {
 
@@ -15,6 +16,8 @@ static thread_local std::string g_err;
 static hipStream_t g_stream = nullptr;
 static int g_device = -1;
 static std::mutex g_mu;
+static std::mutex g_streams_mu;
+static std::unordered_set<hipStream_t> g_streams;  // made by orc_stream_create
 
 int set_error(int code, const std::string& msg) {
     g_err = msg;
@@ -22,6 +25,11 @@ int set_error(int code, const std::string& msg) {
 }
 hipStream_t resolve_stream(orc_stream_t s) { return s ? (hipStream_t)s : g_stream; }
 bool initialized() { return g_device >= 0; }
+bool library_stream(hipStream_t s) {
+    if (s == g_stream) return true;
+    std::lock_guard<std::mutex> lk(g_streams_mu);
+    return g_streams.count(s) != 0;
+}
 
 __global__ void k_fill(uint8_t* p, uint8_t v, size_t n) {
     size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 16;
@@ -141,11 +149,21 @@ extern "C" int orc_stream_create(orc_stream_t* s) {
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
     hipStream_t st;
     ORC_HIP_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    {
+        std::lock_guard<std::mutex> lk(g_streams_mu);
+        g_streams.insert(st);
+    }
     *s = (orc_stream_t)st;
     return ORC_OK;
 }
 extern "C" int orc_stream_destroy(orc_stream_t s) {
-    if (s) ORC_HIP_CHECK(hipStreamDestroy((hipStream_t)s));
+    if (!s) return ORC_OK;
+    {
+        std::lock_guard<std::mutex> lk(g_streams_mu);
+        g_streams.erase((hipStream_t)s);
+    }
+    pf_ws_forget((hipStream_t)s);
+    ORC_HIP_CHECK(hipStreamDestroy((hipStream_t)s));
     return ORC_OK;
 }
 extern "C" int orc_stream_sync(orc_stream_t s) {

@@ -221,3 +221,99 @@ def test_token_chunks(dev, oracle):
     got = _gemm(dev, ty, w, X, n_out)
     pick = np.r_[0:40, 3400:3600]  # both sides of the chunk boundary
     _check(got[pick], X[pick], W)
+
+
+@pytest.mark.parametrize("H,KVH,hd,sp,nt", [(8, 1, 64, 0, 1), (7, 7, 128, 31, 33), (24, 8, 128, 4000, 30),
+                                            (28, 4, 128, 95, 129), (16, 2, 64, 640, 600)])
+def test_prefill_attention(dev, H, KVH, hd, sp, nt):
+    """The prefill attention over split K and V (csrc/orc_attn_pf.hip) against
+    float64: block edges of 32 positions, padded row tiles, key ranges merged
+    over workgroups (few rows over a long cache), values whose scale differs by
+    2^20 between key blocks and dimensions. Scores are fp32-like (2^-22 per
+    product, |score| up to ~30): 4e-6 of the row's largest output. A repeat
+    gives the same bits; the cache rows past the pass are untouched."""
+    print(f"[gpu] pf attention H={H} KVH={KVH} hd={hd} sp={sp} nt={nt}", flush=True)
+    rng = np.random.default_rng(sp + nt)
+    ctx, ld = sp + nt + 40, (H + 2 * KVH) * hd
+    qkv = rng.normal(0, 1, (nt, ld)).astype(np.float32)
+    K, V = (rng.normal(0, 1, (KVH, ctx, hd)).astype(np.float32) for _ in range(2))
+    V *= (2.0 ** rng.integers(-10, 10, (KVH, ctx // 32 + 1))).repeat(32, 1)[:, :ctx, None].astype(np.float32)
+    K[:, :, : hd // 8] *= 2.0 ** -20
+    th = np.arange(ctx)[:, None] / 1e4 ** (np.arange(hd // 2) * 2.0 / hd)
+    tab = np.stack([np.cos(th), np.sin(th)], -1).astype(np.float32)
+    dq, dt, do = dev.upload(qkv), dev.upload(tab), dev.alloc(nt * H * hd * 4)
+    outs = []
+    for _ in range(2):
+        dK, dV = dev.upload(K), dev.upload(V)
+        dev.check(dev.L.orc_attn_prefill(dq.ptr, ld, nt, H, KVH, hd, sp, dt.ptr, dK.ptr, dV.ptr, ctx, do.ptr, H * hd,
+                                         None))
+        outs.append(do.read(np.float32).reshape(nt, H, hd))
+    assert np.array_equal(outs[0], outs[1])
+    got = outs[0]
+    x = qkv.astype(np.float64).reshape(nt, H + 2 * KVH, hd)
+    c, s = (tab[sp:sp + nt, None, :, i].astype(np.float64) for i in range(2))
+
+    def rope(v):
+        a, b = v[..., : hd // 2], v[..., hd // 2:]
+        return np.concatenate([a * c - b * s, a * s + b * c], -1)
+
+    q, k = rope(x[:, :H]), rope(x[:, H:H + KVH])
+    k64, v64 = K.astype(np.float64), V.astype(np.float64)
+    k64[:, sp:sp + nt], v64[:, sp:sp + nt] = k.transpose(1, 0, 2), x[:, H + KVH:].transpose(1, 0, 2)
+    Kc, Vc = dK.read(np.float32).reshape(K.shape), dV.read(np.float32).reshape(V.shape)
+    assert np.allclose(Kc[:, :sp + nt], k64[:, :sp + nt], rtol=1e-6, atol=1e-6)
+    assert np.array_equal(Vc[:, :sp + nt], v64[:, :sp + nt].astype(np.float32))
+    assert np.array_equal(Kc[:, sp + nt:], K[:, sp + nt:]) and np.array_equal(Vc[:, sp + nt:], V[:, sp + nt:])
+    mask = np.arange(sp + nt)[None] > sp + np.arange(nt)[:, None]
+    for h in range(H):
+        g = h // (H // KVH)
+        sc = q[:, h] @ k64[g, :sp + nt].T / np.sqrt(hd)
+        sc[mask] = -np.inf
+        p = np.exp(sc - sc.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        want, scale = p @ v64[g, :sp + nt], p @ np.abs(v64[g, :sp + nt])
+        assert np.all(np.abs(got[:, h] - want) <= 4e-6 * scale.max(1, keepdims=True)), h
+
+
+def test_prefill_attention_captured_and_streams(dev):
+    """A captured call keeps the kernel without the workspace and replays to
+    fp32 rounding of the other; calls on a second stream take the workspace in
+    turn (same bits)."""
+    rng = np.random.default_rng(4)
+    H, KVH, hd, sp, nt = 8, 2, 64, 50, 70
+    ctx, ld = 128, (H + 2 * KVH) * hd
+    qkv = rng.normal(0, 1, (nt, ld)).astype(np.float32)
+    K, V = (rng.normal(0, 1, (KVH, ctx, hd)).astype(np.float32) for _ in range(2))
+    th = np.arange(ctx)[:, None] / 1e4 ** (np.arange(hd // 2) * 2.0 / hd)
+    dt = dev.upload(np.stack([np.cos(th), np.sin(th)], -1).astype(np.float32))
+    dq, dK, dV = dev.upload(qkv), dev.upload(K), dev.upload(V)
+    dos = [dev.alloc(nt * H * hd * 4) for _ in range(5)]
+
+    def run(do, s):
+        dev.check(dev.L.orc_attn_prefill(dq.ptr, ld, nt, H, KVH, hd, sp, dt.ptr, dK.ptr, dV.ptr, ctx, do.ptr, H * hd,
+                                         s))
+
+    s, graph = C.c_void_p(), C.c_void_p()
+    dev.check(dev.L.orc_stream_create(C.byref(s)))
+    run(dos[0], None)
+    dev.sync()
+    want = dos[0].read(np.float32)
+    for i, st in enumerate((s, None, s)):
+        run(dos[1 + i], st)
+    dev.sync()
+    for i in range(3):
+        assert np.array_equal(dos[1 + i].read(np.float32), want), i
+    dev.check(dev.L.orc_graph_begin(s))
+    run(dos[4], s)
+    dev.check(dev.L.orc_graph_end(s, C.byref(graph)))
+    for _ in range(3):
+        dev.check(dev.L.orc_graph_launch(graph, s))
+        run(dos[0], None)
+        dev.sync()
+        assert np.array_equal(dos[0].read(np.float32), want)
+        assert np.allclose(dos[4].read(np.float32), want, rtol=0, atol=4e-6 * np.abs(want).max())
+    dev.check(dev.L.orc_graph_destroy(graph))
+    dev.check(dev.L.orc_stream_destroy(s))
+    run(dos[0], None)  # the workspace's last use was on the destroyed stream or on this one
+    dev.sync()
+    assert np.array_equal(dos[0].read(np.float32), want)
