@@ -340,7 +340,9 @@ int orc_sampler_init(void* d_state, float temperature, float top_p, int top_k, f
                      uint64_t seed, const int32_t* d_hist, int n_hist, orc_stream_t stream);
 /* Sampler::sample (sampler.cpp:91-97) on one row of n_vocab logits: penalty,
  * temperature, softmax, top-k, top-p, draw, record. Like the reference it
- * rewrites the row in place (it ends up holding the probabilities). */
+ * rewrites the row in place (it ends up holding the probabilities). T > 0 and
+ * 1 <= top_k <= 128 on up to 196608 logits run split over many workgroups with
+ * the state's scratch (calls on one state must not overlap). */
 int orc_sample(void* d_state, float* d_logits, int n_vocab, int32_t* d_out, orc_stream_t stream);
 /* Sampler::record (sampler.cpp:99-105) of n device ids, in order. */
 int orc_sampler_record(void* d_state, const int32_t* d_tok, int n, orc_stream_t stream);

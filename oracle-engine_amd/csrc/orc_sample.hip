@@ -1136,6 +1136,26 @@ __device__ int32_t draw_kept(float u, int cut, float total, SampScratch& sh) {
     return tok;
 }
 
+// The draw of Sampler::sample (sampler.cpp:78-85) from the sorted kept set
+// sh.cand[0 .. sh.bcast[4]) (at most kTxK) of mass sh.fb[0]: r = u * mass, r
+// -= p down the set, the first one if rounding leaves r > 0. One wave, the
+// entries passed between lanes.
+__device__ int32_t draw_sorted(float u, SampScratch& sh) {
+    const int lane = threadIdx.x & 63, cut = sh.bcast[4];
+    const unsigned long long ea = lane < cut ? sh.cand[lane] : 0ull, eb = lane + 64 < cut ? sh.cand[lane + 64] : 0ull;
+    float r = u * sh.fb[0];
+    int32_t tok = (int32_t)(rdlane(ea, 0) & 0xFFFFFFFFu);
+    for (int i = 0; i < cut; ++i) {
+        const unsigned long long c = i < 64 ? rdlane(ea, i) : rdlane(eb, i - 64);
+        r -= cand_p(c);
+        if (r <= 0.f) {
+            tok = (int32_t)(c & 0xFFFFFFFFu);
+            break;
+        }
+    }
+    return tok;
+}
+
 // The kept set sh.cand[0 .. sh.bcast[4]) (at most kTxK) and its mass
 // sh.fb[0] into the state's list of row r.
 __device__ void keep_list(TxWork& w, int r, SampScratch& sh) {
@@ -1153,13 +1173,36 @@ __device__ void keep_list(TxWork& w, int r, SampScratch& sh) {
 // The split transform's last step for row blockIdx.x. MODE 0: p written;
 // 1: p written and one draw from it into out[0] (and out2[0]); 2 (list): the
 // kept set, its mass and size go to the state's scratch for
-// k_accept_engine, p is not written.
+// k_accept_engine, p is not written; 3 (sample, one row): workgroup 0 draws
+// as Sampler::sample does (r = u * mass, r -= p down the sorted set,
+// sampler.cpp:78-85), records and writes the id to out[0], workgroup 1 + g
+// turns slice g of the row into its probabilities (what the reference leaves
+// there).
 template <int MODE>
 __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int ld, int n, float* p, int ldp,
                                                    int32_t* out, int32_t* out2) {
-    constexpr bool DRAW = MODE == 1, LIST = MODE == 2;
+    constexpr bool DRAW = MODE == 1, LIST = MODE == 2, SAMPLE = MODE == 3;
     __shared__ SampScratch sh;
-    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int r = SAMPLE ? 0 : blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    if (SAMPLE && blockIdx.x > 0) {
+        const TxWork& w = s->tx;
+        if (!tx_split(s) || w.ovf[0]) return;  // workgroup 0 rewrites the whole row
+        const int G = gridDim.x - 1, b = (blockIdx.x - 1) * kTxSlice, e = min(n, b + kTxSlice);
+        float mx = lane < G ? w.mx[0][lane] : -INFINITY, sum = lane < G ? w.sum[0][lane] : 0.f;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = lg[min(b + tid + j * kST, n - 1)];
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+            sum += __shfl_xor(sum, o, 64);
+        }
+        const float inv_s = 1.f / sum;  // e and 1 / sum as the candidates' p
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (b + tid + j * kST < e) lg[b + tid + j * kST] = expf(v[j] - mx) * inv_s;
+        return;
+    }
     float* prow = p + (size_t)r * ldp;
     int32_t tok = -1;
     if (tx_split(s)) {
@@ -1169,12 +1212,16 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
         const int ncv = lane < G ? w.nc[r][lane] : 0;
         const bool ovf = w.ovf[r] != 0;
         if (tid == 0 && !ovf) {  // through LDS, so both are read before the merge's first barrier
-            sh.fb[2] = DRAW ? mt_canonical(s) : 0.f;
+            sh.fb[2] = DRAW || SAMPLE ? mt_canonical(s) : 0.f;
             sh.fb[3] = s->top_p;
         }
         if (ovf) {
             const int k = topk_sorted(s, lg + (size_t)r * ld, n, sh, true);
-            if (LIST) {
+            if (SAMPLE) {
+                topp_cut(s, nullptr, k, sh);
+                if (tid == 0) sh.fb[2] = mt_canonical(s);
+                __syncthreads();
+            } else if (LIST) {
                 topp_cut(s, nullptr, k, sh);
                 __syncthreads();
                 keep_list(w, r, sh);
@@ -1270,7 +1317,7 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
             const float total = sh.fb[0];
             if (LIST) {
                 keep_list(w, r, sh);
-            } else {
+            } else if (!SAMPLE) {
                 for (int i = tid; i < cut; i += kST) {
                     const int id = (int)(sh.cand[i] & 0xFFFFFFFFu);
                     prow[id] = cand_p(sh.cand[i]) / total;
@@ -1278,6 +1325,18 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
             }
             if (DRAW) tok = draw_kept(sh.fb[2], cut, total, sh);
         }
+        if (SAMPLE) {  // the sorted kept set is sh.cand[0 .. cut), its mass sh.fb[0]
+            if (tid < 64) tok = draw_sorted(sh.fb[2], sh);
+        }
+    } else if (SAMPLE) {
+        tok = sample_row(s, lg, n, sh);
+    }
+    if (SAMPLE) {
+        if (tid == 0) {
+            record_tok(s, tok);  // sampler.cpp:95
+            *out = tok;
+        }
+        return;
     }
     if (DRAW) {
         if (tok < 0) {  // the transform was the one-workgroup one: draw over the row as k_draw does
@@ -1592,6 +1651,18 @@ using namespace orc;
 // (kCandMax). The state itself is device memory the host never reads back.
 static std::mutex g_all_mu;
 static std::unordered_set<const void*> g_all_tokens;
+// And of those whose parameters the split transform does not take (T <= 0,
+// top_k 0 or above kTxK): orc_sample gives them the one-workgroup kernel at
+// once. Only a hint: either route samples any state as its parameters say.
+static std::unordered_set<const void*> g_one_wg;
+
+static void note_params(const void* d_state, float temperature, int top_k) {
+    std::lock_guard<std::mutex> lk(g_all_mu);
+    if (top_k == 0 && temperature > 0.f) g_all_tokens.insert(d_state);  // T <= 0 sorts nothing (argmax)
+    else g_all_tokens.erase(d_state);
+    if (temperature > 0.f && top_k >= 1 && top_k <= kTxK) g_one_wg.erase(d_state);
+    else g_one_wg.insert(d_state);
+}
 
 static int check_vocab(const void* d_state, int n_vocab, const char* who) {
     if (n_vocab <= kCandMax) return ORC_OK;
@@ -1632,11 +1703,7 @@ extern "C" int orc_sampler_init(void* d_state, float temperature, float top_p, i
     if (!d_state || repeat_last < 0 || repeat_last >= kSampHist || n_hist < 0 || (n_hist && !d_hist) ||
         top_k < 0 || top_k > kCandMax)
         return set_error(ORC_E_INVALID, "sampler_init: bad args (0 <= top_k <= 16384, 0 <= repeat_last < 4096)");
-    {
-        std::lock_guard<std::mutex> lk(g_all_mu);
-        if (top_k == 0 && temperature > 0.f) g_all_tokens.insert(d_state);  // T <= 0 sorts nothing (argmax)
-        else g_all_tokens.erase(d_state);
-    }
+    note_params(d_state, temperature, top_k);
     hipLaunchKernelGGL(k_sampler_init, dim3(1), dim3(64), 0, resolve_stream(s), (DevSampler*)d_state,
                        (uint32_t)seed, temperature, top_p, repeat_penalty, top_k, repeat_last, d_hist, n_hist);
     ORC_LAUNCH_CHECK();
@@ -1648,11 +1715,7 @@ extern "C" int orc_sampler_set_params(void* d_state, float temperature, float to
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
     if (!d_state || repeat_last < 0 || repeat_last >= kSampHist || top_k < 0 || top_k > kCandMax)
         return set_error(ORC_E_INVALID, "sampler_set_params: bad args (0 <= top_k <= 16384, 0 <= repeat_last < 4096)");
-    {
-        std::lock_guard<std::mutex> lk(g_all_mu);
-        if (top_k == 0 && temperature > 0.f) g_all_tokens.insert(d_state);  // T <= 0 sorts nothing (argmax)
-        else g_all_tokens.erase(d_state);
-    }
+    note_params(d_state, temperature, top_k);
     hipLaunchKernelGGL(k_sampler_set, dim3(1), dim3(64), 0, resolve_stream(s), (DevSampler*)d_state, 1, temperature,
                        top_p, repeat_penalty, top_k, repeat_last);
     ORC_LAUNCH_CHECK();
@@ -1672,8 +1735,26 @@ extern "C" int orc_sample(void* d_state, float* d_logits, int n_vocab, int32_t* 
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
     if (!d_state || !d_logits || !d_out || n_vocab <= 0) return set_error(ORC_E_INVALID, "sample: bad args");
     if (int rc = check_vocab(d_state, n_vocab, "sample")) return rc;
-    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kST), 0, resolve_stream(s), (DevSampler*)d_state, d_logits, n_vocab,
-                       d_out);
+    const hipStream_t st = resolve_stream(s);
+    DevSampler* ds = (DevSampler*)d_state;
+    bool one_wg;
+    {
+        std::lock_guard<std::mutex> lk(g_all_mu);
+        one_wg = g_one_wg.count(d_state) != 0;
+    }
+    // three launches over the row's slices (152064 logits, top_k 40: 240 us in
+    // one workgroup, 28 split; 1024 logits 78 and 20)
+    if (!one_wg && tx_shape(n_vocab, 1)) {
+        const int G = (n_vocab + kTxSlice - 1) / kTxSlice;
+        hipLaunchKernelGGL(k_tx_max<true>, dim3(G), dim3(kST), 0, st, ds, d_logits, n_vocab, n_vocab,
+                           (const int32_t*)nullptr, 0, (float*)nullptr, 0);
+        hipLaunchKernelGGL(k_tx_exp, dim3(G), dim3(kST), 0, st, ds, (const float*)d_logits, n_vocab, n_vocab,
+                           (float*)nullptr, 0);
+        hipLaunchKernelGGL(k_tx_final<3>, dim3(1 + G), dim3(kST), 0, st, ds, d_logits, n_vocab, n_vocab,
+                           (float*)nullptr, 0, d_out, (int32_t*)nullptr);
+    } else {
+        hipLaunchKernelGGL(k_sample, dim3(1), dim3(kST), 0, st, ds, d_logits, n_vocab, d_out);
+    }
     ORC_LAUNCH_CHECK();
     return ORC_OK;
 }
