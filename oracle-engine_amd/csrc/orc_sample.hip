@@ -7,9 +7,11 @@
 // written out as distributions, feeds the min(1, p/q) acceptance chain with
 // residual resampling (no reference counterpart).
 //
-// One 1024-thread workgroup samples one row of logits, in place as the
-// reference does (the row ends up holding the probabilities); the transform
-// and the acceptance chain also run split over many workgroups (below):
+// The row is sampled in place as the reference does (it ends up holding the
+// probabilities). For T > 0 and 1 <= top_k <= kTxK the transform, and with it
+// orc_sample, runs split over many workgroups (below), as does the acceptance
+// chain; other parameters take one 1024-thread workgroup per row (k_sample,
+// k_transform), with the same steps:
 //  * repeat penalty over the device-resident history, one entry at a time
 //    (repeated ids compound), then temperature (skipped for T <= 0 or 1);
 //  * T <= 0: first index of the maximum;
@@ -323,6 +325,9 @@ __device__ __forceinline__ unsigned long long rdlane(unsigned long long v, int i
     const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)v, i);
     const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(v >> 32), i);
     return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ double rdlane(double v, int i) {
+    return __builtin_bit_cast(double, rdlane(__builtin_bit_cast(unsigned long long, v), i));
 }
 
 // The parameters the split transform takes (T > 0, 1 <= top_k <= kTxK).
@@ -840,18 +845,25 @@ __global__ __launch_bounds__(kST) void k_draw(DevSampler* s, const float* p, int
 //             slice maximum;
 //  k_tx_exp   (slice x row): e = expf(l - row max) as the one-workgroup
 //             softmax forms it, slice sum, and the slice's candidates: every
-//             e >= t (1 - 2^-20), t found by a radix search on the bits of e
-//             such that at least min(top_k, positives) of the slice's e are
-//             >= t. Any e below that bound has top_k others in its slice whose
-//             p = e / sum is strictly larger, since both products are normal
-//             floats rounded once and differ by more than two roundings, so
-//             the row's top_k by (p desc, index asc) are all candidates;
-//  k_tx_final (row): p = e * (1 / sum of the slice sums); a radix search
-//             over the candidates' p down to a prefix the k-th largest p has
-//             and at most max(k, 64) candidates reach; those sorted by (p
-//             desc, index asc), the first k kept, top-p cut, p_out written;
-//             optionally one draw from it. (Below t = 2^-100 the slice passes
-//             every positive e on: p could then be subnormal.)
+//             e >= t (1 - 2^-20), t such that at least min(top_k, positives)
+//             of the slice's e are >= t (group_bound; if that passes on more
+//             than kTxStop, a radix search on the bits of e). Any e below
+//             that bound has top_k others in its slice whose p = e / sum is
+//             strictly larger, since both products are normal floats rounded
+//             once and differ by more than two roundings, so the row's top_k
+//             by (p desc, index asc) are all candidates;
+//  k_tx_final (row): p = e * (1 / sum of the slice sums); the candidates a
+//             second bound of the same kind leaves, sorted by (p desc, index
+//             asc), the first k kept, top-p cut, p_out written; optionally
+//             one draw from it. (Below t = 2^-100 the slice passes every
+//             positive e on: p could then be subnormal.)
+// Bound by latency (one row is 0.6 MB): launches, the memory round trips
+// before the first barrier, and barriers of sixteen waves. A 152064-token row,
+// top_k 40, with radix searches on LDS counters in both kernels and serial
+// loops for the cut and the draw -> with the group maxima and lane_chain:
+// k_tx_exp 9.5 -> 5.2 us, k_tx_final 17.9 -> 10.4 us with a draw and 11.5 ->
+// 7.8 without; a round of six proposals with its verify rows and chain 247 ->
+// 167 us, orc_sample 28.4 -> 20.8 us.
 // Zero e (exp underflow) never enters: zero-probability candidates change
 // neither the kept mass nor a draw. Other parameters (T <= 0, top_k 0 or
 // above kTxK) take the one-workgroup transform in k_tx_max's first
@@ -971,33 +983,107 @@ __device__ int radix_step(int want, int& above, unsigned int& prefix, unsigned i
     return ge;
 }
 
+// A cheap bound for the want-th largest of a workgroup's keys (32-bit, 0 for
+// none): the keys fall into kST / 8 groups, those of eight neighbouring lanes,
+// and with at least `want` groups whose maximum is >= t at least that many
+// keys are. group_max leaves the group maxima in gm; group_bound (a barrier
+// after it) returns the want-th largest of them with its low bits cleared, as
+// every wave finds it by itself, or 0 if fewer groups hold a key. Of random
+// keys in random places about groups ln(1 / (1 - want / groups)) reach the
+// bound: 48 for top_k 40, 89 for 64, so up to kTxBound it takes one barrier
+// and no counters where the radix search takes three to five passes of LDS
+// counters, most of one workgroup's keys on the same few. Beyond that, and
+// for keys that lie together, the radix search's bound is the tighter one (a
+// slice passes kTxStop on). A round of four proposals, bound against search:
+// 153 / 181 us at top_k 65 and 189 / 198 at 90 (152064 logits), 154 / 171 and
+// 198 / 183 (32000); at 128, 238 / 223 and 220 / 205.
+constexpr int kTxBound = 72;
+__device__ __forceinline__ void group_max(unsigned int key, unsigned int* gm) {
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) key = max(key, (unsigned int)__shfl_xor((int)key, o, 64));
+    if ((threadIdx.x & 7) == 0) gm[threadIdx.x >> 3] = key;
+}
+__device__ __forceinline__ unsigned int group_bound(int want, const unsigned int* gm) {
+    static_assert(kST / 8 == 128, "two group maxima per lane");
+    const int lane = threadIdx.x & 63;
+    const unsigned int a = gm[lane], b = gm[lane + 64];
+    unsigned int t = 0;
+#pragma unroll
+    for (int bit = 30; bit >= 14; --bit) {  // sign clear; the low mantissa bits do not matter to a bound
+        const unsigned int c = t | (1u << bit);
+        if (__popcll(__ballot(a >= c)) + __popcll(__ballot(b >= c)) >= want) t = c;
+    }
+    return t;
+}
+
+// Places for the items a workgroup keeps (NI per thread): each wave's count
+// goes to cnt; after the barrier total() is theirs, and slot(j) the place of
+// this thread's item j (kept ones only).
+template <int NI> struct Place {
+    unsigned long long m[NI];
+    int base, total;
+    __device__ __forceinline__ void count(const bool (&keep)[NI], int* cnt) {
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            m[j] = __ballot(keep[j]);
+            c += __popcll(m[j]);
+        }
+        if ((threadIdx.x & 63) == 0) cnt[threadIdx.x >> 6] = c;
+    }
+    __device__ __forceinline__ void finish(const int* cnt) {
+        static_assert(kST / 64 == 16, "sixteen waves");
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        int inc = cnt[lane & 15];  // inclusive scan over sixteen lanes
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            const int t = __shfl_up(inc, o, 16);
+            if ((lane & 15) >= o) inc += t;
+        }
+        total = __shfl(inc, 15, 64);
+        base = wave ? __shfl(inc, wave - 1, 64) : 0;
+    }
+    __device__ __forceinline__ int slot(int j) const {
+        int c = base;
+#pragma unroll
+        for (int i = 0; i < j; ++i) c += __popcll(m[i]);
+        return c + __builtin_amdgcn_mbcnt_hi((unsigned int)(m[j] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)m[j], 0));
+    }
+};
+
 __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, int ld, int n, float* p, int ldp) {
     if (!tx_split(s)) return;
-    __shared__ unsigned int wc[2 * 16 * 16];
+    __shared__ unsigned int wc[2 * 16 * 16], gm[kST / 8];
     __shared__ float red[kST / 64];
-    __shared__ int ired[kST / 64], slots;
+    __shared__ int ired[kST / 64], cnt[2][kST / 64];
     const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, G = gridDim.x;
     TxWork& w = s->tx;
-    float mx = lane < G ? w.mx[r][lane] : -INFINITY;  // G <= 64: one slice maximum per lane
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    const int b = g * kTxSlice, e = min(n, b + kTxSlice);
+    const int b = g * kTxSlice, e = min(n, b + kTxSlice), top_k = s->top_k;
     const float* row = lg + (size_t)r * ld;
     float* prow = p + (size_t)r * ldp;
     float ev[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ev[j] = row[min(b + tid + j * kST, n - 1)];
+    float mx = lane < G ? w.mx[r][lane] : -INFINITY;  // G <= 64: one slice maximum per lane
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     float sum = 0.f;
     int npos = 0;  // positive e, + 2^16 x those below 2^-31 (top key nibble under 3)
+    unsigned int top = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int i = b + tid + j * kST;
-        ev[j] = 0.f;
         if (i < e) {
-            ev[j] = expf(row[i] - mx);
+            ev[j] = expf(ev[j] - mx);
             if (p) prow[i] = 0.f;
             sum += ev[j];
             npos += ev[j] > 0.f ? (ev[j] < 0x1p-31f ? 0x10001 : 1) : 0;
+            if (ev[j] > 0.f) top = max(top, __builtin_bit_cast(unsigned int, ev[j]));
+        } else {
+            ev[j] = 0.f;
         }
     }
+    group_max(top, gm);
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         sum += __shfl_xor(sum, o, 64);
@@ -1007,7 +1093,6 @@ __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, 
         red[tid >> 6] = sum;
         ired[tid >> 6] = npos;
     }
-    if (tid == 0) slots = 0;
     __syncthreads();
     npos = 0;
     for (int i = 0; i < kST / 64; ++i) npos += ired[i];
@@ -1018,38 +1103,51 @@ __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, 
         for (int i = 1; i < kST / 64; ++i) t += red[i];  // fixed order
         w.sum[r][g] = t;
     }
-    const int want = min(s->top_k, npos);
-    unsigned int prefix = 0, mask = 0;
+    const int want = min(top_k, npos);
+    Place<4> at;
+    at.total = 0;
     if (want > 0) {
         const int stop = max(want, kTxStop);  // candidates the slice may pass on
-        int above = 0;
-        if (nib3) {
-            prefix = 0x30000000u;
-            mask = 0xF0000000u;
-        }
-        for (int shift = nib3 ? 24 : 28; shift >= 0; shift -= 4) {
-            unsigned int* buf = radix_buf(wc, shift);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                radix_count(__builtin_bit_cast(unsigned int, ev[j]), ev[j] > 0.f, mask, prefix, shift, buf);
-            if (radix_step(want, above, prefix, mask, shift, wc) <= stop) break;
-        }
+        bool keep[4];
         // bound: 2^-20 below the threshold; below 2^-100 every positive e
         // (p = e / sum could then be subnormal, where rounding is not relative)
-        const float t = __builtin_bit_cast(float, prefix);
-        const float tm = t < 0x1p-100f ? 0.f : t * (1.f - 0x1p-20f);
+        auto pass_on = [&](unsigned int key, int* c) {
+            const float t = __builtin_bit_cast(float, key);
+            const float tm = t < 0x1p-100f ? 0.f : t * (1.f - 0x1p-20f);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) keep[j] = ev[j] > 0.f && ev[j] >= tm;
+            at.count(keep, c);
+            __syncthreads();
+            at.finish(c);
+        };
+        if (want <= kTxBound) pass_on(group_bound(want, gm), cnt[0]);
+        if (want > kTxBound || at.total > stop) {
+            unsigned int prefix = 0, mask = 0;
+            int above = 0;
+            if (nib3) {
+                prefix = 0x30000000u;
+                mask = 0xF0000000u;
+            }
+            for (int shift = nib3 ? 24 : 28; shift >= 0; shift -= 4) {
+                unsigned int* buf = radix_buf(wc, shift);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    radix_count(__builtin_bit_cast(unsigned int, ev[j]), ev[j] > 0.f, mask, prefix, shift, buf);
+                if (radix_step(want, above, prefix, mask, shift, wc) <= stop) break;
+            }
+            pass_on(prefix, cnt[1]);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (ev[j] > 0.f && ev[j] >= tm) {
-                const int slot = atomicAdd(&slots, 1);
+            if (keep[j]) {
+                const int slot = at.slot(j);
                 if (slot < kTxCand)
                     w.cand[r][g][slot] = make_uint2(__builtin_bit_cast(unsigned int, ev[j]), (unsigned int)(b + tid + j * kST));
             }
     }
-    __syncthreads();
     if (tid == 0) {
-        w.nc[r][g] = min(slots, kTxCand);
-        if (slots > kTxCand) w.ovf[r] = 1;
+        w.nc[r][g] = min(at.total, kTxCand);
+        if (at.total > kTxCand) w.ovf[r] = 1;
     }
 }
 
@@ -1060,10 +1158,38 @@ __device__ void rank_sort(const unsigned long long* src, unsigned long long* dst
     if (tid < m) {
         const unsigned long long k = src[tid];
         int rank = 0;
+#pragma unroll 8
         for (int j = 0; j < m; ++j) rank += src[j] < k;
         dst[rank] = k;
     }
     __syncthreads();
+}
+
+// The running values of one serial chain over up to 128 entries held two per
+// lane (entry i < 64: lane i's a, else lane i - 64's b; zeros past n): starting
+// from v, each entry is added (SUB: taken off) in order, and the value after
+// entry i is left with its lane in ra / rb. Nothing but the additions is
+// serial (the choice of an entry is a ballot over the lanes afterwards), so an
+// entry costs one dependent add instead of a compare and a branch as well.
+template <bool SUB, class T> __device__ __forceinline__ T lane_chain(T v, T a, T b, int n, T& ra, T& rb) {
+    const int lane = threadIdx.x & 63;
+    auto half = [&](T x, int n0, T& r) {
+        for (int i0 = 0; i0 < n0; i0 += 8)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const T e = rdlane(x, i0 + i);
+                v = SUB ? v - e : v + e;
+                r = lane == i0 + i ? v : r;
+            }
+    };
+    half(a, min(n, 64), ra);
+    half(b, n - 64, rb);
+    return v;
+}
+// the first entry of a ballot pair over such entries, or `none`
+__device__ __forceinline__ int first_entry(bool a, bool b, int none) {
+    const unsigned long long ma = __ballot(a), mb = __ballot(b);
+    return ma ? __ffsll(ma) - 1 : mb ? __ffsll(mb) + 63 : none;
 }
 
 // topp_cut on wave 0 for k <= 128 candidates: the same running float sum in
@@ -1074,19 +1200,12 @@ __device__ void topp_cut_wave(float top_p, int k, SampScratch& sh) {
     if (tid < 64) {
         const float a = tid < k ? cand_p(sh.cand[tid]) : 0.f;
         const float b = tid + 64 < k ? cand_p(sh.cand[tid + 64]) : 0.f;
-        float cum = 0.f;
-        int cut = k;
-        for (int i = 0; i < k; ++i) {
-            cum += i < 64 ? rdlane(a, i) : rdlane(b, i - 64);
-            if (cum >= top_p) {
-                cut = i + 1;
-                break;
-            }
-        }
-        if (tid == 0) {
-            sh.bcast[4] = cut;
-            sh.fb[0] = cum;  // the kept mass: the same sum over the first cut
-        }
+        float ca = 0.f, cb = 0.f;
+        const float all = lane_chain<false>(0.f, a, b, k, ca, cb);
+        const int at = first_entry(tid < k && ca >= top_p, tid + 64 < k && cb >= top_p, k);
+        if (tid == 0) sh.bcast[4] = min(at + 1, k);
+        // the kept mass: the same sum over the first cut
+        if (at == k ? tid == 0 : (at & 63) == tid) sh.fb[0] = at == k ? all : at < 64 ? ca : cb;
     }
     __syncthreads();
 }
@@ -1094,46 +1213,36 @@ __device__ void topp_cut_wave(float top_p, int k, SampScratch& sh) {
 // One draw from the kept set sh.cand[0 .. cut) (p_out[id] = p / total), as
 // k_draw does over the whole row: u * (sum of p_out in index order, double),
 // first index where the running sum reaches it, the last one if rounding
-// leaves it short. The set is put in index order first. Whole workgroup.
+// leaves it short. The set is put in index order first. Whole workgroup, the
+// result on its first wave.
 __device__ int32_t draw_kept(float u, int cut, float total, SampScratch& sh) {
-    const int tid = threadIdx.x;
-    unsigned long long* byid = (unsigned long long*)sh.dscan;  // (index, p_out bits), kST entries
-    unsigned long long* src = byid + kST / 2;
-    static_assert(kTxK <= kST / 2, "kept set fits half of the scan buffer");
-    if (tid < cut) {
-        const unsigned long long c = sh.cand[tid];
-        const float pv = cand_p(c) / total;
-        src[tid] = ((c & 0xFFFFFFFFull) << 32) | __builtin_bit_cast(unsigned int, pv);
-    }
-    __syncthreads();
-    rank_sort(src, byid, cut);
-    if (tid < 64) {  // wave 0, the entries passed between lanes
-        const unsigned long long ea = tid < cut ? byid[tid] : 0ull, eb = tid + 64 < cut ? byid[tid + 64] : 0ull;
-        auto entry = [&](int i) { return i < 64 ? rdlane(ea, i) : rdlane(eb, i - 64); };
-        double tot = 0.0;
-        for (int i = 0; i < cut; ++i) {
-            const float pv = __builtin_bit_cast(float, (unsigned int)entry(i));
-            if (pv > 0.f) tot += (double)pv;
-        }
-        double rr = (double)u * tot;
-        int tok = -1, last = -1;
-        for (int i = 0; i < cut; ++i) {
-            const unsigned long long c = entry(i);
-            const float pv = __builtin_bit_cast(float, (unsigned int)c);
-            if (!(pv > 0.f)) continue;
-            last = (int)(c >> 32);
-            rr -= (double)pv;
-            if (rr <= 0.0) {
-                tok = last;
-                break;
-            }
-        }
-        if (tid == 0) sh.bcast[3] = tok >= 0 ? tok : max(last, 0);
-    }
-    __syncthreads();
-    const int32_t tok = sh.bcast[3];
-    __syncthreads();
-    return tok;
+    static_assert(kTxK <= 128, "two entries per lane");
+    if (threadIdx.x >= 64) return 0;
+    const int lane = threadIdx.x;
+    unsigned long long* byid = (unsigned long long*)sh.dscan;  // (index, p_out bits) by index
+    auto place = [&](int i) {
+        if (i >= cut) return;
+        const unsigned long long c = sh.cand[i];
+        const unsigned int id = (unsigned int)c;
+        int rank = 0;
+#pragma unroll 8
+        for (int j = 0; j < cut; ++j) rank += (unsigned int)sh.cand[j] < id;
+        byid[rank] = ((unsigned long long)id << 32) | __builtin_bit_cast(unsigned int, cand_p(c) / total);
+    };
+    place(lane);
+    if (cut > 64) place(lane + 64);
+    // one wave: its LDS operations complete in order
+    const unsigned long long ea = lane < cut ? byid[lane] : 0ull, eb = lane + 64 < cut ? byid[lane + 64] : 0ull;
+    const float pa = __builtin_bit_cast(float, (unsigned int)ea), pb = __builtin_bit_cast(float, (unsigned int)eb);
+    const double da = pa > 0.f ? (double)pa : 0.0, db = pb > 0.f ? (double)pb : 0.0;
+    double ra = 0.0, rb = 0.0;
+    const double tot = lane_chain<false>(0.0, da, db, cut, ra, rb);
+    lane_chain<true>((double)u * tot, da, db, cut, ra, rb);
+    const int at = first_entry(pa > 0.f && ra <= 0.0, pb > 0.f && rb <= 0.0, -1);
+    if (at >= 0) return (int32_t)((at < 64 ? rdlane(ea, at) : rdlane(eb, at - 64)) >> 32);
+    const unsigned long long ma = __ballot(pa > 0.f), mb = __ballot(pb > 0.f);
+    if (mb) return (int32_t)(rdlane(eb, 63 - __clzll(mb)) >> 32);
+    return ma ? (int32_t)(rdlane(ea, 63 - __clzll(ma)) >> 32) : 0;
 }
 
 // The draw of Sampler::sample (sampler.cpp:78-85) from the sorted kept set
@@ -1142,18 +1251,12 @@ __device__ int32_t draw_kept(float u, int cut, float total, SampScratch& sh) {
 // entries passed between lanes.
 __device__ int32_t draw_sorted(float u, SampScratch& sh) {
     const int lane = threadIdx.x & 63, cut = sh.bcast[4];
-    const unsigned long long ea = lane < cut ? sh.cand[lane] : 0ull, eb = lane + 64 < cut ? sh.cand[lane + 64] : 0ull;
-    float r = u * sh.fb[0];
-    int32_t tok = (int32_t)(rdlane(ea, 0) & 0xFFFFFFFFu);
-    for (int i = 0; i < cut; ++i) {
-        const unsigned long long c = i < 64 ? rdlane(ea, i) : rdlane(eb, i - 64);
-        r -= cand_p(c);
-        if (r <= 0.f) {
-            tok = (int32_t)(c & 0xFFFFFFFFu);
-            break;
-        }
-    }
-    return tok;
+    const unsigned long long none = 0xFFFFFFFF00000000ull;  // p 0, id 0
+    const unsigned long long ea = lane < cut ? sh.cand[lane] : none, eb = lane + 64 < cut ? sh.cand[lane + 64] : none;
+    float ra = 0.f, rb = 0.f;
+    lane_chain<true>(u * sh.fb[0], cand_p(ea), cand_p(eb), cut, ra, rb);
+    const int at = first_entry(lane < cut && ra <= 0.f, lane + 64 < cut && rb <= 0.f, 0);
+    return (int32_t)((at < 64 ? rdlane(ea, at) : rdlane(eb, at - 64)) & 0xFFFFFFFFu);
 }
 
 // The kept set sh.cand[0 .. sh.bcast[4]) (at most kTxK) and its mass
@@ -1205,16 +1308,24 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
     }
     float* prow = p + (size_t)r * ldp;
     int32_t tok = -1;
+    TxWork& w = s->tx;
+    const int G = (n + kTxSlice - 1) / kTxSlice;
+    const int wave = tid >> 6;
+    const float sv = lane < G ? w.sum[r][lane] : 0.f;  // loads issued together, before the branches below
+    const int ncv = lane < G ? w.nc[r][lane] : 0;
+    // wave w takes the candidates of slices w, w + 16, ...; the first 64
+    // of each come without waiting for their number
+    constexpr int kGS = kTxMaxG / (kST / 64), kNS = kTxCand / 64;
+    static_assert(kGS * (kST / 64) == kTxMaxG && kNS * 64 == kTxCand, "whole waves");
+    uint2 c[kGS][kNS];
+#pragma unroll
+    for (int i = 0; i < kGS; ++i) {
+        const int g = wave + i * (kST / 64);
+        c[i][0] = g < G ? w.cand[r][g][lane] : make_uint2(0, 0);
+    }
+    const bool ovf = w.ovf[r] != 0;
+    const int k = min(s->top_k, n);
     if (tx_split(s)) {
-        TxWork& w = s->tx;
-        const int G = (n + kTxSlice - 1) / kTxSlice;
-        const float sv = lane < G ? w.sum[r][lane] : 0.f;  // loads issued together
-        const int ncv = lane < G ? w.nc[r][lane] : 0;
-        const bool ovf = w.ovf[r] != 0;
-        if (tid == 0 && !ovf) {  // through LDS, so both are read before the merge's first barrier
-            sh.fb[2] = DRAW || SAMPLE ? mt_canonical(s) : 0.f;
-            sh.fb[3] = s->top_p;
-        }
         if (ovf) {
             const int k = topk_sorted(s, lg + (size_t)r * ld, n, sh, true);
             if (SAMPLE) {
@@ -1234,80 +1345,101 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
             const float inv_s = 1.f / sum;
-            int* off = (int*)sh.dscan;  // off[0 .. G]: exclusive prefix of the slice counts
-            if (tid == 0) sh.bcast[6] = 0;  // set when a candidate's p is below 2^-31
-            if (tid < 64) {
-                const int c = ncv;
-                int inc = c;  // inclusive scan over the wave
+            // keys ~bits(p) << 32 | index (p desc, index asc); none: all ones
+            unsigned long long key[kGS * kNS];
+            unsigned int top = 0;
+            bool low = false;  // a p below 2^-31
+            int N = ncv;
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int t = __shfl_up(inc, o, 64);
-                    if (tid >= o) inc += t;
-                }
-                if (tid <= G) off[tid] = inc - c;
-            }
-            __syncthreads();
-            const int N = off[G];
-            // gather, wave w taking slices w, w + 16, ...: key = ~bits(p) << 32 |
-            // index (p desc, index asc)
-            for (int g = tid >> 6; g < G; g += kST / 64) {
-                const int c0 = off[g], nc = off[g + 1] - c0;
+            for (int o = 32; o >= 1; o >>= 1) N += __shfl_xor(N, o, 64);
 #pragma unroll
-                for (int j = lane; j < kTxCand; j += 64)
-                    if (j < nc) {
-                        const uint2 c = w.cand[r][g][j];
-                        const float pv = __builtin_bit_cast(float, c.x) * inv_s;
-                        if (pv < 0x1p-31f) sh.bcast[6] = 1;
-                        sh.cand[c0 + j] = ((unsigned long long)(~__builtin_bit_cast(unsigned int, pv)) << 32) | c.y;
+            for (int i = 0; i < kGS; ++i) {
+                const int g = wave + i * (kST / 64), nc = g < G ? __builtin_amdgcn_readlane(ncv, g) : 0;
+#pragma unroll
+                for (int j = 0; j < kNS; ++j) {
+                    key[i * kNS + j] = ~0ull;
+                    if (j > 0 && 64 * j < nc) c[i][j] = w.cand[r][g][64 * j + lane];
+                    if (64 * j + lane < nc) {
+                        const float pv = __builtin_bit_cast(float, c[i][j].x) * inv_s;
+                        const unsigned int pb = __builtin_bit_cast(unsigned int, pv);
+                        low |= pv < 0x1p-31f;
+                        top = max(top, pb);
+                        key[i * kNS + j] = ((unsigned long long)(~pb) << 32) | c[i][j].y;
                     }
+                }
             }
+            unsigned int* gm = sh.hist;
+            static_assert(kST / 8 <= 512, "group maxima in the counters");
+            group_max(top, gm);
             __syncthreads();
-            // a prefix of p bits that the k-th largest p has and at most
-            // max(k, kRank) candidates reach (the k-th largest itself when ties
-            // leave more)
-            const int k = min(s->top_k, n);
+            // thr: bits of a p that at least min(k, N) candidates reach. With it
+            // every candidate of the row's top k has p >= thr: sorted, the first
+            // k of them are the ones the one-workgroup transform sorts first.
+            // From the group maxima where about as many candidates reach it as
+            // are wanted, else (nothing near the bound, or ties) from a radix
+            // search down to a prefix that at most max(k, kRank) reach.
             const int want = min(k, N);
-            constexpr int kRank = 64;
-            unsigned int prefix = 0, mask = 0;
-            int above = 0;
-            if (N > max(want, kRank)) {
-                const bool nib3 = sh.bcast[6] == 0;  // p <= 1: key nibble 3 unless p < 2^-31
-                if (nib3) {
-                    prefix = 0x30000000u;
-                    mask = 0xF0000000u;
+            constexpr int kRank = 64, kDirect = 256;
+            unsigned long long* sel = (unsigned long long*)sh.dscan;
+            Place<kGS * kNS> at;
+            bool keep[kGS * kNS];
+            auto select = [&](unsigned int thr, int* cnt) {
+#pragma unroll
+                for (int j = 0; j < kGS * kNS; ++j)
+                    keep[j] = key[j] != ~0ull && ~(unsigned int)(key[j] >> 32) >= thr;
+                at.count(keep, cnt);
+                __syncthreads();
+                at.finish(cnt);
+            };
+            auto put = [&](unsigned long long* d, int cap) {
+#pragma unroll
+                for (int j = 0; j < kGS * kNS; ++j)
+                    if (keep[j]) {
+                        const int slot = at.slot(j);
+                        if (slot < cap) d[slot] = key[j];
+                    }
+            };
+            at.total = 0;
+            if (want <= kTxBound) select(N <= kDirect ? 0u : group_bound(want, gm), sh.ired);
+            if (want > kTxBound || at.total > kDirect) {
+                unsigned int prefix = 0, mask = 0;
+                int above = 0;
+                if (N > max(want, kRank)) {
+                    const bool nib3 = !__syncthreads_or(low);  // p <= 1: key nibble 3 unless p < 2^-31
+                    if (nib3) {
+                        prefix = 0x30000000u;
+                        mask = 0xF0000000u;
+                    }
+                    for (int shift = nib3 ? 24 : 28; shift >= 0; shift -= 4) {
+                        unsigned int* buf = radix_buf(sh.hist, shift);
+#pragma unroll
+                        for (int j = 0; j < kGS * kNS; ++j)
+                            radix_count(~(unsigned int)(key[j] >> 32), key[j] != ~0ull, mask, prefix, shift, buf);
+                        if (radix_step(want, above, prefix, mask, shift, sh.hist) <= max(want, kRank)) break;
+                    }
                 }
-                for (int shift = nib3 ? 24 : 28; shift >= 0; shift -= 4) {
-                    unsigned int* buf = radix_buf(sh.hist, shift);
-                    for (int i = tid; i < N; i += kST)
-                        radix_count(~(unsigned int)(sh.cand[i] >> 32), true, mask, prefix, shift, buf);
-                    if (radix_step(want, above, prefix, mask, shift, sh.hist) <= max(want, kRank)) break;
-                }
+                __syncthreads();  // readers of the last counts are done
+                select(prefix, sh.ired);
             }
-            // every candidate of the row's top k has p >= thr; sorted, the first
-            // k of them are the ones the one-workgroup transform sorts first
-            const unsigned int thr = prefix;
-            if (tid == 0) sh.bcast[2] = 0;
-            __syncthreads();
-            unsigned long long* sel = (unsigned long long*)sh.dscan + 32;  // after off[]
-            constexpr int kSel = kST - 32;
-            static_assert((kTxMaxG + 1) * sizeof(int) <= 32 * sizeof(double), "offsets before the selection");
-            for (int i = tid; i < N; i += kST) {
-                const unsigned long long c = sh.cand[i];
-                if (~(unsigned int)(c >> 32) >= thr) {
-                    const int slot = atomicAdd(&sh.bcast[2], 1);
-                    if (slot < kSel) sel[slot] = c;
+            const int m0 = at.total;
+            // the uniform and top_p through the LDS, by a wave the sort leaves idle
+            auto scalars = [&] {
+                if (tid == kST - 64) {
+                    sh.fb[2] = DRAW || SAMPLE ? mt_canonical(s) : 0.f;
+                    sh.fb[3] = s->top_p;
                 }
-            }
-            __syncthreads();
-            const int m0 = sh.bcast[2];
-            if (m0 <= kSel) {
+            };
+            if (m0 <= kST) {
+                put(sel, kST);
+                __syncthreads();
+                scalars();
                 rank_sort(sel, sh.cand, m0);
-            } else {  // many ties at the threshold: sort the whole candidate list
-                for (int i = tid; i < N; i += kST)
-                    if (~(unsigned int)(sh.cand[i] >> 32) < thr) sh.cand[i] = ~0ull;
+            } else {  // many ties at the threshold: sort them all
+                put(sh.cand, kCandMax);
                 int mp = 1;
-                while (mp < N) mp <<= 1;
-                for (int i = N + tid; i < mp; i += kST) sh.cand[i] = ~0ull;
+                while (mp < m0) mp <<= 1;
+                for (int i = m0 + tid; i < mp; i += kST) sh.cand[i] = ~0ull;
+                scalars();
                 __syncthreads();
                 bitonic_sort(sh, mp);
             }
