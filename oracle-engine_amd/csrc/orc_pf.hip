@@ -865,7 +865,13 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
 // 3B and 7B layer matrices at 20 to 1023 tokens (us, MI355X; rows x n_in,
 // type, tokens):
 //  * 128 rows x 32 tokens for at most 32 tokens (7B gate+up Q6_K 75 against
-//    90 with 64-token tiles);
+//    90 with 64-token tiles), and for narrow matrices, where 64-token tiles in
+//    the most ranges below leave CUs idle: such a launch is one wave per SIMD
+//    and as long as its chain of dependent products, which a 32-token tile
+//    halves (896 x 896 Q8_0 in four ranges: 14.0 at 64 tokens, 16.0 at 256
+//    and 19.4 at 512 against 20.4, 28.6 and 28.9 with 64-token tiles; 1023
+//    tokens, one range, 24.9 against 30.4; 896 x 4864 at 256 27.5 against
+//    30.0; 3072 x 3072 Q4_K at 48 19.7 against 20.9);
 //  * 128 x 128 once such tiles are two per CU (7B gate+up, 1023 tokens: 891
 //    against 1024 with 128 x 64; 2048-wide Q4_0 216 against 270) and K is at
 //    least eight superblocks (0.5B gate+up, n_in 896: 110 against 87), not
@@ -874,7 +880,9 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
 //  * 128 x 64 otherwise (3072 x 3072 Q4_K, 1023 tokens: 84 against 107).
 //  * K is split while the tiles leave CUs idle: up to 768 workgroups, ranges
 //    of at least two superblocks (three above 128 tokens, where the partial
-//    sums weigh more): 3584 x 18944 at 127 tokens 364 in one range, 106 in
+//    sums weigh more); with 32-token tiles up to 512 workgroups, and a short
+//    K in up to four ranges (896 x 896 at 256 tokens: 22.6, 18.6, 17.6 and
+//    16.1 in one to four). 3584 x 18944 at 127 tokens 364 in one range, 106 in
 //    eight; 3584 x 3584 83 -> 38; F16 2048 x 8192 142 -> 34. F16 and BF16
 //    rows are cut at 16 superblocks at any size: the rounding of one long
 //    chain would exceed the fp32 kernel's (8192 values: 1.35e-7 of the
@@ -887,11 +895,14 @@ static PfPlan pf_plan(int type, const QmvParams& p, int supers) {
     const bool dense = type == ORC_F16 || type == ORC_BF16;
     auto wgs = [&](int bt) { return (long)((rows + 127) / 128) * ((p.n_tok + bt - 1) / bt); };
     PfPlan r{1, 1};
-    if (p.n_tok <= 32) r.shape = 2;
-    else if (type != ORC_BF16 && p.n_tok > 64 && supers >= 8 && wgs(128) >= 2 * g_n_cu) r.shape = 0;
-    const long w = wgs(r.shape == 0 ? 128 : r.shape == 1 ? 64 : 32), want = 3 * g_n_cu;
     const int most = std::min(16, std::max(1, (supers + 1) / (p.n_tok <= 128 ? 2 : 3)));
-    r.nz = (int)std::max<long>(1, std::min<long>(most, want / w));
+    if (p.n_tok <= 32 || wgs(64) * most < g_n_cu) r.shape = 2;
+    else if (type != ORC_BF16 && p.n_tok > 64 && supers >= 8 && wgs(128) >= 2 * g_n_cu) r.shape = 0;
+    if (r.shape == 2)
+        r.nz = (int)std::min<long>(std::max(most, std::min(supers, 4)), 2 * g_n_cu / wgs(32));
+    else
+        r.nz = (int)std::min<long>(most, 3 * g_n_cu / wgs(r.shape == 0 ? 128 : 64));
+    r.nz = std::max(r.nz, 1);
     if (dense) r.nz = std::max(r.nz, (supers + 15) / 16);
     return r;
 }

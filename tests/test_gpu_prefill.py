@@ -317,3 +317,18 @@ def test_prefill_attention_captured_and_streams(dev):
     run(dos[0], None)  # the workspace's last use was on the destroyed stream or on this one
     dev.sync()
     assert np.array_equal(dos[0].read(np.float32), want)
+
+
+# narrow matrices above 32 tokens (32-token tiles, a short K in up to four
+# ranges): one and several ranges, ragged tokens and rows, and on both sides
+# of the line to 64-token tiles (256 workgroups of those: 16 row blocks here)
+@pytest.mark.parametrize("qt,nt,n_out,n_in", [(ol.Q8_0, 33, 896, 896), (ol.Q8_0, 257, 129, 896), (ol.Q8_0, 1023, 896, 896),
+                                              (ol.Q4_0, 512, 33, 96), (ol.Q4_K, 48, 3072, 3072), (ol.Q6_K, 97, 130, 1280),
+                                              (ol.BF16, 190, 96, 1024), (ol.F16, 95, 31, 4352), (ol.Q8_0, 1024, 2048, 64),
+                                              (ol.Q8_0, 960, 2048, 64)])
+def test_narrow_matrices(dev, oracle, qt, nt, n_out, n_in):
+    print(f"[gpu] pf narrow type={qt} nt={nt} {n_out}x{n_in}", flush=True)
+    rng = np.random.default_rng(nt + n_in)
+    w, ty, W = _weights(dev, oracle, qt, n_out, n_in, rng)
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    _check(_gemm(dev, ty, w, X, n_out), X, W)
