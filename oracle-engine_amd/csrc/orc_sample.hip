@@ -54,9 +54,8 @@ constexpr int kTxK = 128;          // largest top_k of the split path
 
 struct TxWork {
     float mx[kTxRows][kTxMaxG];   // slice maxima of the scaled logits
-    float sum[kTxRows][kTxMaxG];  // slice sums of exp(l - max)
-    int nc[kTxRows][kTxMaxG];     // candidates per slice
-    int ovf[kTxRows];             // a slice had more than kTxCand candidates
+    float sum[kTxRows][kTxMaxG];  // slice sums of exp(l - slice maximum)
+    int nc[kTxRows][kTxMaxG];     // candidates per slice (more than kTxCand: not all were passed on)
     int cut[kTxRows];             // kept set of each row (list mode)
     float total[kTxRows];         // its mass
     uint2 kept[kTxRows][kTxK];    // (index, bits of p), sorted by (p desc, index asc)
@@ -65,7 +64,7 @@ struct TxWork {
     float ch_u;
     double ch_sum[kTxMaxG];  // slice sums of the draw's weights
     int ch_last[kTxMaxG];    // last positive weight of each slice (-1: none)
-    uint2 cand[kTxRows][kTxMaxG][kTxCand];  // (bits of exp(l - max), index)
+    uint2 cand[kTxRows][kTxMaxG][kTxCand];  // (bits of the scaled logit, index)
 };
 
 struct DevSampler {
@@ -695,7 +694,7 @@ __global__ void k_sampler_record(DevSampler* s, const int32_t* tok, int n) {
 // reference loop), [3] 1 if all drafts were accepted and the bonus emitted,
 // [4 ..] the emitted ids. With d_pos / d_next the device round state advances.
 // With split set and the split transform's parameters, the rows' kept sets
-// were written by k_tx_max<true> / k_tx_exp / k_tx_final<2> (row i's window
+// were written by k_tx_slice<true> / k_tx_final<2> (row i's window
 // assumes proposals 0 .. i-1 accepted, the only case in which row i is
 // sampled) and wave 0 draws from them: r = u * mass, r -= p down the sorted
 // set, the first candidate if rounding leaves r > 0 (sampler.cpp:78-85).
@@ -840,99 +839,44 @@ __global__ __launch_bounds__(kST) void k_draw(DevSampler* s, const float* p, int
 // ── the transform split over workgroups ─────────────────────────────────────
 // Same results as transform_row (same kept set; the softmax sum is added in
 // another order, so p may differ in its last bit) for T > 0 and
-// 1 <= top_k <= kTxK, in three launches:
-//  k_tx_max   (slice x row): repeat penalty of the ids in the slice, 1/T,
-//             slice maximum;
-//  k_tx_exp   (slice x row): e = expf(l - row max) as the one-workgroup
-//             softmax forms it, slice sum, and the slice's candidates: every
-//             e >= t (1 - 2^-20), t such that at least min(top_k, positives)
-//             of the slice's e are >= t (group_bound; if that passes on more
-//             than kTxStop, a radix search on the bits of e). Any e below
-//             that bound has top_k others in its slice whose p = e / sum is
-//             strictly larger, since both products are normal floats rounded
-//             once and differ by more than two roundings, so the row's top_k
-//             by (p desc, index asc) are all candidates;
-//  k_tx_final (row): p = e * (1 / sum of the slice sums); the candidates a
+// 1 <= top_k <= kTxK, in two launches:
+//  k_tx_slice (slice x row): repeat penalty of the ids in the slice, 1/T,
+//             slice maximum m, the sum of e' = expf(l - m), and the slice's
+//             candidates: every e' >= t (1 - 2^-15), t such that at least
+//             min(top_k, positives) of the slice's e' are >= t (group_bound;
+//             if that passes on more than kTxStop, a radix search on the bits
+//             of e');
+//  k_tx_final (row): the row maximum M, the row sum over the slices' sums
+//             times exp(m - M) (in double: the factor is exact to the fp32
+//             sums), e = expf(l - M) and p = e * (1 / sum) of the candidates
+//             as the one-workgroup softmax forms them; the candidates a
 //             second bound of the same kind leaves, sorted by (p desc, index
 //             asc), the first k kept, top-p cut, p_out written; optionally
-//             one draw from it. (Below t = 2^-100 the slice passes every
-//             positive e on: p could then be subnormal.)
+//             one draw from it.
+// Any e' below its slice's bound has top_k others in the slice whose logits
+// are more than 2^-15.1 larger. For p >= 2^-100, |l - M| is below 128, where a
+// difference is rounded by at most 2^-18: their p is strictly larger, so the
+// row's top_k by (p desc, index asc) are all candidates. Below 2^-100 the p of
+// different logits may tie, and a row whose k-th p lies there is redone by
+// the one-workgroup transform where its p are written out. Where it is only
+// drawn from it is not: such entries, at most 2^-82 of the largest p, change
+// neither the kept mass nor r.
+// The row maximum used to be a launch of its own in front of the slices'.
 // Bound by latency (one row is 0.6 MB): launches, the memory round trips
 // before the first barrier, and barriers of sixteen waves. A 152064-token row,
-// top_k 40, with radix searches on LDS counters in both kernels and serial
-// loops for the cut and the draw -> with the group maxima and lane_chain:
-// k_tx_exp 9.5 -> 5.2 us, k_tx_final 17.9 -> 10.4 us with a draw and 11.5 ->
-// 7.8 without; a round of six proposals with its verify rows and chain 247 ->
-// 167 us, orc_sample 28.4 -> 20.8 us.
+// top_k 40, k_tx_final with radix searches on LDS counters and serial loops
+// for the cut and the draw -> with the group maxima and lane_chain: 17.9 ->
+// 10.4 us with a draw and 11.5 -> 7.8 without.
+// Without the separate maximum launch a round of six proposals with its verify
+// rows and chain went from 168 to 158 us (247 before all of it), orc_sample
+// from 20.7 to 18.9.
 // Zero e (exp underflow) never enters: zero-probability candidates change
-// neither the kept mass nor a draw. Other parameters (T <= 0, top_k 0 or
-// above kTxK) take the one-workgroup transform in k_tx_max's first
-// workgroup of each row, and a row with a slice of more than kTxCand
-// candidates (ties) is redone by that transform in k_tx_final from the
-// scaled logits the first launch left in the row.
-
-// ENG (the Engine rule's rows, list mode): row r's window is the history
-// plus extra[0], extra[0], ..., extra[r-1], extra[r-1] (the proposals an
-// accepted prefix records twice each); other parameters are left to the
-// one-workgroup acceptance kernel.
-template <bool ENG>
-__global__ __launch_bounds__(kST) void k_tx_max(DevSampler* s, float* lg, int ld, int n, const int32_t* extra,
-                                                 int extra_base, float* p, int ldp) {
-    __shared__ SampScratch sh;
-    const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
-    float* row = lg + (size_t)r * ld;
-    if (!tx_split(s)) {
-        if (!ENG && g == 0) transform_row(s, row, n, extra, extra_base + r, p + (size_t)r * ldp, sh);
-        return;
-    }
-    const int b = g * kTxSlice, e = min(n, b + kTxSlice);
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int i = b + tid + j * kST;
-        v[j] = i < e ? row[i] : -INFINITY;
-    }
-    if (s->pen > 1.f) {
-        // sampler.cpp:15-27: each occurrence of an id in the window divides
-        // (l > 0) or multiplies its logit by the penalty, in window order; an
-        // id's value sees only its own occurrences, so applying them c times
-        // in a row is the same sequence of operations.
-        int* hits = (int*)sh.cand;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hits[tid + j * kST] = 0;
-        __syncthreads();
-        const int L = s->nh + (ENG ? 2 * r : extra_base + r);
-        const int start = L - s->last > 0 ? L - s->last : 0;
-        for (int q = start + tid; q < L; q += kST) {
-            const int32_t id = q < s->nh ? s->hist[q] : extra[(q - s->nh) >> (ENG ? 1 : 0)];
-            if (id >= b && id < e) atomicAdd(&hits[id - b], 1);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            for (int c = hits[tid + j * kST]; c > 0; --c) v[j] = v[j] > 0.f ? v[j] / s->pen : v[j] * s->pen;
-    }
-    const float T = s->temp;
-    if (T != 1.f) {
-        const float inv_t = 1.f / T;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] *= inv_t;
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int i = b + tid + j * kST;
-        if (i < e) {
-            row[i] = v[j];
-            mx = fmaxf(mx, v[j]);
-        }
-    }
-    mx = block_max(mx, sh);
-    if (tid == 0) {
-        s->tx.mx[r][g] = mx;
-        if (g == 0) s->tx.ovf[r] = 0;
-    }
-}
+// neither the kept mass nor a draw, and neither does a slice all of whose e
+// are zero, however many of its logits tie (a mask of the lowest value).
+// Other parameters (T <= 0, top_k 0 or above kTxK) take the one-workgroup
+// transform in k_tx_final, and so does a row with a slice of more than
+// kTxCand candidates (ties), from the scaled logits the first launch left in
+// the row.
 
 // Radix steps over a workgroup, 4-bit digits: each wave counts its keys'
 // digits into its own 16 counters of one half of wc (2 x 16 x 16 LDS
@@ -1051,37 +995,82 @@ template <int NI> struct Place {
     }
 };
 
-__global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, int ld, int n, float* p, int ldp) {
+// ENG (the Engine rule's rows, list mode): row r's window is the history
+// plus extra[0], extra[0], ..., extra[r-1], extra[r-1] (the proposals an
+// accepted prefix records twice each); other parameters are left to the
+// one-workgroup acceptance kernel.
+template <bool ENG>
+__global__ __launch_bounds__(kST) void k_tx_slice(DevSampler* s, float* lg, int ld, int n, const int32_t* extra,
+                                                  int extra_base, float* p, int ldp) {
     if (!tx_split(s)) return;
+    __shared__ int hits[kTxSlice];
     __shared__ unsigned int wc[2 * 16 * 16], gm[kST / 8];
-    __shared__ float red[kST / 64];
+    __shared__ float red[kST / 64], mred[kST / 64];
     __shared__ int ired[kST / 64], cnt[2][kST / 64];
-    const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, G = gridDim.x;
+    const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     TxWork& w = s->tx;
     const int b = g * kTxSlice, e = min(n, b + kTxSlice), top_k = s->top_k;
-    const float* row = lg + (size_t)r * ld;
+    float* row = lg + (size_t)r * ld;
     float* prow = p + (size_t)r * ldp;
-    float ev[4];
+    float v[4], ev[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ev[j] = row[min(b + tid + j * kST, n - 1)];
-    float mx = lane < G ? w.mx[r][lane] : -INFINITY;  // G <= 64: one slice maximum per lane
+    for (int j = 0; j < 4; ++j) {
+        const int i = b + tid + j * kST;
+        v[j] = i < e ? row[i] : -INFINITY;
+    }
+    if (s->pen > 1.f) {
+        // sampler.cpp:15-27: each occurrence of an id in the window divides
+        // (l > 0) or multiplies its logit by the penalty, in window order; an
+        // id's value sees only its own occurrences, so applying them c times
+        // in a row is the same sequence of operations.
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    float sum = 0.f;
-    int npos = 0;  // positive e, + 2^16 x those below 2^-31 (top key nibble under 3)
-    unsigned int top = 0;
+        for (int j = 0; j < 4; ++j) hits[tid + j * kST] = 0;
+        __syncthreads();
+        const int L = s->nh + (ENG ? 2 * r : extra_base + r);
+        const int start = L - s->last > 0 ? L - s->last : 0;
+        for (int q = start + tid; q < L; q += kST) {
+            const int32_t id = q < s->nh ? s->hist[q] : extra[(q - s->nh) >> (ENG ? 1 : 0)];
+            if (id >= b && id < e) atomicAdd(&hits[id - b], 1);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            for (int c = hits[tid + j * kST]; c > 0; --c) v[j] = v[j] > 0.f ? v[j] / s->pen : v[j] * s->pen;
+    }
+    const float T = s->temp;
+    if (T != 1.f) {
+        const float inv_t = 1.f / T;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] *= inv_t;
+    }
+    float mx = -INFINITY;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int i = b + tid + j * kST;
         if (i < e) {
-            ev[j] = expf(ev[j] - mx);
+            row[i] = v[j];
             if (p) prow[i] = 0.f;
-            sum += ev[j];
-            npos += ev[j] > 0.f ? (ev[j] < 0x1p-31f ? 0x10001 : 1) : 0;
-            if (ev[j] > 0.f) top = max(top, __builtin_bit_cast(unsigned int, ev[j]));
-        } else {
-            ev[j] = 0.f;
+            mx = fmaxf(mx, v[j]);
         }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) mred[tid >> 6] = mx;
+    __syncthreads();
+    mx = mred[lane & 15];
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    const float m0 = mx == -INFINITY ? 0.f : mx;  // nothing but -inf (and NaN) in the slice: e' = 0 (NaN)
+    float sum = 0.f;
+    int npos = 0;  // positive e', + 2^16 x those below 2^-31 (top key nibble under 3)
+    unsigned int top = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = b + tid + j * kST;
+        ev[j] = i < e ? expf(v[j] - m0) : 0.f;
+        sum += ev[j];
+        npos += ev[j] > 0.f ? (ev[j] < 0x1p-31f ? 0x10001 : 1) : 0;
+        if (ev[j] > 0.f) top = max(top, __builtin_bit_cast(unsigned int, ev[j]));
     }
     group_max(top, gm);
 #pragma unroll
@@ -1096,12 +1085,13 @@ __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, 
     __syncthreads();
     npos = 0;
     for (int i = 0; i < kST / 64; ++i) npos += ired[i];
-    const bool nib3 = (npos >> 16) == 0;  // every positive e has key nibble 3 (2^-31 <= e <= 1)
+    const bool nib3 = (npos >> 16) == 0;  // every positive e' has key nibble 3 (2^-31 <= e' <= 1)
     npos &= 0xFFFF;
     if (tid == 0) {
         float t = red[0];
         for (int i = 1; i < kST / 64; ++i) t += red[i];  // fixed order
         w.sum[r][g] = t;
+        w.mx[r][g] = mx;
     }
     const int want = min(top_k, npos);
     Place<4> at;
@@ -1109,11 +1099,11 @@ __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, 
     if (want > 0) {
         const int stop = max(want, kTxStop);  // candidates the slice may pass on
         bool keep[4];
-        // bound: 2^-20 below the threshold; below 2^-100 every positive e
-        // (p = e / sum could then be subnormal, where rounding is not relative)
+        // bound: 2^-15 below the threshold; below 2^-100 every positive e'
+        // (the threshold's relative step is lost among subnormals)
         auto pass_on = [&](unsigned int key, int* c) {
             const float t = __builtin_bit_cast(float, key);
-            const float tm = t < 0x1p-100f ? 0.f : t * (1.f - 0x1p-20f);
+            const float tm = t < 0x1p-100f ? 0.f : t * (1.f - 0x1p-15f);
 #pragma unroll
             for (int j = 0; j < 4; ++j) keep[j] = ev[j] > 0.f && ev[j] >= tm;
             at.count(keep, c);
@@ -1142,13 +1132,26 @@ __global__ __launch_bounds__(kST) void k_tx_exp(DevSampler* s, const float* lg, 
             if (keep[j]) {
                 const int slot = at.slot(j);
                 if (slot < kTxCand)
-                    w.cand[r][g][slot] = make_uint2(__builtin_bit_cast(unsigned int, ev[j]), (unsigned int)(b + tid + j * kST));
+                    w.cand[r][g][slot] = make_uint2(__builtin_bit_cast(unsigned int, v[j]), (unsigned int)(b + tid + j * kST));
             }
     }
-    if (tid == 0) {
-        w.nc[r][g] = min(at.total, kTxCand);
-        if (at.total > kTxCand) w.ovf[r] = 1;
-    }
+    if (tid == 0) w.nc[r][g] = at.total;
+}
+
+// What the slices of a row left, one slice per lane (G <= 64): the row maximum
+// M, 1 / the row's sum, and the slice's candidates nc (0 where all its e are
+// zero); returns whether a slice had more than it could pass on. Every wave
+// forms the same values.
+__device__ __forceinline__ bool tx_gather(float mx, float sum, int& nc, float& M, float& inv_s) {
+    M = mx;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    double t = sum == 0.f && mx < M ? 0.0 : (double)sum * exp((double)mx - (double)M);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o, 64);
+    inv_s = 1.f / (float)t;
+    if (!(expf(mx - M) > 0.f)) nc = 0;
+    return __any(nc > kTxCand);
 }
 
 // Sorts the m <= kST distinct keys src[0 .. m) ascending into dst by rank
@@ -1283,24 +1286,21 @@ __device__ void keep_list(TxWork& w, int r, SampScratch& sh) {
 // there).
 template <int MODE>
 __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int ld, int n, float* p, int ldp,
-                                                   int32_t* out, int32_t* out2) {
+                                                   const int32_t* extra, int extra_base, int32_t* out, int32_t* out2) {
     constexpr bool DRAW = MODE == 1, LIST = MODE == 2, SAMPLE = MODE == 3;
     __shared__ SampScratch sh;
     const int r = SAMPLE ? 0 : blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     if (SAMPLE && blockIdx.x > 0) {
+        if (!tx_split(s)) return;  // workgroup 0 rewrites the whole row
         const TxWork& w = s->tx;
-        if (!tx_split(s) || w.ovf[0]) return;  // workgroup 0 rewrites the whole row
         const int G = gridDim.x - 1, b = (blockIdx.x - 1) * kTxSlice, e = min(n, b + kTxSlice);
-        float mx = lane < G ? w.mx[0][lane] : -INFINITY, sum = lane < G ? w.sum[0][lane] : 0.f;
+        const float mxv = lane < G ? w.mx[0][lane] : -INFINITY, sv = lane < G ? w.sum[0][lane] : 0.f;
+        int ncv = lane < G ? w.nc[0][lane] : 0;
+        float mx, inv_s;
+        if (tx_gather(mxv, sv, ncv, mx, inv_s)) return;  // so it does here
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = lg[min(b + tid + j * kST, n - 1)];
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-            sum += __shfl_xor(sum, o, 64);
-        }
-        const float inv_s = 1.f / sum;  // e and 1 / sum as the candidates' p
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (b + tid + j * kST < e) lg[b + tid + j * kST] = expf(v[j] - mx) * inv_s;
@@ -1312,7 +1312,8 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
     const int G = (n + kTxSlice - 1) / kTxSlice;
     const int wave = tid >> 6;
     const float sv = lane < G ? w.sum[r][lane] : 0.f;  // loads issued together, before the branches below
-    const int ncv = lane < G ? w.nc[r][lane] : 0;
+    const float mxv = lane < G ? w.mx[r][lane] : -INFINITY;
+    int ncv = lane < G ? w.nc[r][lane] : 0;
     // wave w takes the candidates of slices w, w + 16, ...; the first 64
     // of each come without waiting for their number
     constexpr int kGS = kTxMaxG / (kST / 64), kNS = kTxCand / 64;
@@ -1323,10 +1324,12 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
         const int g = wave + i * (kST / 64);
         c[i][0] = g < G ? w.cand[r][g][lane] : make_uint2(0, 0);
     }
-    const bool ovf = w.ovf[r] != 0;
     const int k = min(s->top_k, n);
+    float u0 = -1.f;  // a uniform already drawn
     if (tx_split(s)) {
-        if (ovf) {
+        float M, inv_s;
+        bool redo = tx_gather(mxv, sv, ncv, M, inv_s);
+        auto one_wg = [&] {
             const int k = topk_sorted(s, lg + (size_t)r * ld, n, sh, true);
             if (SAMPLE) {
                 topp_cut(s, nullptr, k, sh);
@@ -1339,17 +1342,13 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
             } else {
                 write_kept(s, k, prow, n, false, sh);
             }
-        } else {
-            // the row sum over the slice sums (fixed order), as every wave forms it
-            float sum = sv;
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-            const float inv_s = 1.f / sum;
+        };
+        if (!redo) {
             // keys ~bits(p) << 32 | index (p desc, index asc); none: all ones
             unsigned long long key[kGS * kNS];
             unsigned int top = 0;
             bool low = false;  // a p below 2^-31
-            int N = ncv;
+            int N = ncv;  // candidates, those whose e is zero (left out below) among them
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) N += __shfl_xor(N, o, 64);
 #pragma unroll
@@ -1360,11 +1359,13 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
                     key[i * kNS + j] = ~0ull;
                     if (j > 0 && 64 * j < nc) c[i][j] = w.cand[r][g][64 * j + lane];
                     if (64 * j + lane < nc) {
-                        const float pv = __builtin_bit_cast(float, c[i][j].x) * inv_s;
+                        const float ev = expf(__builtin_bit_cast(float, c[i][j].x) - M), pv = ev * inv_s;
                         const unsigned int pb = __builtin_bit_cast(unsigned int, pv);
-                        low |= pv < 0x1p-31f;
-                        top = max(top, pb);
-                        key[i * kNS + j] = ((unsigned long long)(~pb) << 32) | c[i][j].y;
+                        if (ev > 0.f) {
+                            low |= pv < 0x1p-31f;
+                            top = max(top, pb);
+                            key[i * kNS + j] = ((unsigned long long)(~pb) << 32) | c[i][j].y;
+                        }
                     }
                 }
             }
@@ -1372,7 +1373,8 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
             static_assert(kST / 8 <= 512, "group maxima in the counters");
             group_max(top, gm);
             __syncthreads();
-            // thr: bits of a p that at least min(k, N) candidates reach. With it
+            // thr: bits of a p that at least min(k, N) candidates reach (0 where
+            // fewer than that are positive). With it
             // every candidate of the row's top k has p >= thr: sorted, the first
             // k of them are the ones the one-workgroup transform sorts first.
             // From the group maxima where about as many candidates reach it as
@@ -1447,7 +1449,12 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
             topp_cut_wave(sh.fb[3], kk, sh);
             const int cut = sh.bcast[4];
             const float total = sh.fb[0];
-            if (LIST) {
+            // a k-th p below 2^-100: slices may have kept back others of the same p
+            redo = (MODE == 0 || DRAW) && kk == k && cand_p(sh.cand[kk - 1]) < 0x1p-100f;
+            if (redo) {
+                u0 = sh.fb[2];
+                __syncthreads();
+            } else if (LIST) {
                 keep_list(w, r, sh);
             } else if (!SAMPLE) {
                 for (int i = tid; i < cut; i += kST) {
@@ -1455,13 +1462,16 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
                     prow[id] = cand_p(sh.cand[i]) / total;
                 }
             }
-            if (DRAW) tok = draw_kept(sh.fb[2], cut, total, sh);
+            if (DRAW && !redo) tok = draw_kept(sh.fb[2], cut, total, sh);
         }
+        if (redo) one_wg();
         if (SAMPLE) {  // the sorted kept set is sh.cand[0 .. cut), its mass sh.fb[0]
             if (tid < 64) tok = draw_sorted(sh.fb[2], sh);
         }
     } else if (SAMPLE) {
         tok = sample_row(s, lg, n, sh);
+    } else if (!LIST) {
+        transform_row(s, lg + (size_t)r * ld, n, extra, extra_base + r, prow, sh);
     }
     if (SAMPLE) {
         if (tid == 0) {
@@ -1472,7 +1482,8 @@ __global__ __launch_bounds__(kST) void k_tx_final(DevSampler* s, float* lg, int 
     }
     if (DRAW) {
         if (tok < 0) {  // the transform was the one-workgroup one: draw over the row as k_draw does
-            const float u = lane0_uniform(s, sh);
+            __syncthreads();
+            const float u = u0 >= 0.f ? u0 : lane0_uniform(s, sh);
             const double tt = block_total(prow, n, sh);
             tok = block_pick(n, [&](int i) { return prow[i]; }, (double)u * tt, sh);
         }
@@ -1816,16 +1827,11 @@ static void launch_tx(DevSampler* st, float* lg, int ld, int n, int rows, const 
                       float* p, int ldp, int32_t* out, int32_t* out2, hipStream_t s) {
     const dim3 grid((n + kTxSlice - 1) / kTxSlice, rows);
     if (p)
-        hipLaunchKernelGGL(k_tx_max<false>, grid, dim3(kST), 0, s, st, lg, ld, n, extra, extra_base, p, ldp);
+        hipLaunchKernelGGL(k_tx_slice<false>, grid, dim3(kST), 0, s, st, lg, ld, n, extra, extra_base, p, ldp);
     else
-        hipLaunchKernelGGL(k_tx_max<true>, grid, dim3(kST), 0, s, st, lg, ld, n, extra, 0, p, ldp);
-    hipLaunchKernelGGL(k_tx_exp, grid, dim3(kST), 0, s, st, (const float*)lg, ld, n, p, ldp);
-    if (!p)
-        hipLaunchKernelGGL(k_tx_final<2>, dim3(rows), dim3(kST), 0, s, st, lg, ld, n, p, ldp, out, out2);
-    else if (out)
-        hipLaunchKernelGGL(k_tx_final<1>, dim3(rows), dim3(kST), 0, s, st, lg, ld, n, p, ldp, out, out2);
-    else
-        hipLaunchKernelGGL(k_tx_final<0>, dim3(rows), dim3(kST), 0, s, st, lg, ld, n, p, ldp, out, out2);
+        hipLaunchKernelGGL(k_tx_slice<true>, grid, dim3(kST), 0, s, st, lg, ld, n, extra, 0, p, ldp);
+    const auto fin = p ? (out ? k_tx_final<1> : k_tx_final<0>) : k_tx_final<2>;
+    hipLaunchKernelGGL(fin, dim3(rows), dim3(kST), 0, s, st, lg, ld, n, p, ldp, extra, extra_base, out, out2);
 }
 
 extern "C" int orc_sampler_init(void* d_state, float temperature, float top_p, int top_k, float repeat_penalty,
@@ -1874,16 +1880,14 @@ extern "C" int orc_sample(void* d_state, float* d_logits, int n_vocab, int32_t* 
         std::lock_guard<std::mutex> lk(g_all_mu);
         one_wg = g_one_wg.count(d_state) != 0;
     }
-    // three launches over the row's slices (152064 logits, top_k 40: 240 us in
-    // one workgroup, 28 split; 1024 logits 78 and 20)
+    // two launches over the row's slices (152064 logits, top_k 40: 240 us in
+    // one workgroup, 18.9 split)
     if (!one_wg && tx_shape(n_vocab, 1)) {
         const int G = (n_vocab + kTxSlice - 1) / kTxSlice;
-        hipLaunchKernelGGL(k_tx_max<true>, dim3(G), dim3(kST), 0, st, ds, d_logits, n_vocab, n_vocab,
+        hipLaunchKernelGGL(k_tx_slice<true>, dim3(G), dim3(kST), 0, st, ds, d_logits, n_vocab, n_vocab,
                            (const int32_t*)nullptr, 0, (float*)nullptr, 0);
-        hipLaunchKernelGGL(k_tx_exp, dim3(G), dim3(kST), 0, st, ds, (const float*)d_logits, n_vocab, n_vocab,
-                           (float*)nullptr, 0);
         hipLaunchKernelGGL(k_tx_final<3>, dim3(1 + G), dim3(kST), 0, st, ds, d_logits, n_vocab, n_vocab,
-                           (float*)nullptr, 0, d_out, (int32_t*)nullptr);
+                           (float*)nullptr, 0, (const int32_t*)nullptr, 0, d_out, (int32_t*)nullptr);
     } else {
         hipLaunchKernelGGL(k_sample, dim3(1), dim3(kST), 0, st, ds, d_logits, n_vocab, d_out);
     }
