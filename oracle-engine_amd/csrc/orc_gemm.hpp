@@ -73,8 +73,9 @@ void pf_release();
 // split values (83 MB) with room for partial sums, or the split K and V of
 // 32 K positions of eight 128-wide kv heads. pf_ws_takes: whether `bytes` fit
 // and the stream is not being captured. pf_ws_begin locks it and orders the
-// stream behind its last use (kPfBusy: that was on a stream being captured
-// now; the caller takes a path without it); pf_ws_end ends the use and
+// stream behind its last use (kPfBusy: that was on a library stream whose
+// capture was begun through HIP itself instead of orc_graph_begin; the caller
+// takes a path without it); pf_ws_end ends the use and
 // unlocks. pf_ws_forget: a library stream is about to be destroyed.
 constexpr size_t kPfWorkBytes = (size_t)256 << 20;
 constexpr int kPfBusy = 1;

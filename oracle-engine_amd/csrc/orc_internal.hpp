@@ -14,9 +14,10 @@ hipStream_t resolve_stream(orc_stream_t s);
 bool initialized();
 // Whether s is the default stream or one made by orc_stream_create.
 bool library_stream(hipStream_t s);
-// A library stream is about to be destroyed (the prefill workspace's last use
-// may be on it).
+// The prefill workspace's last use may be on a library stream s that is about
+// to be destroyed, or to be captured (pf_ws_capture begins the capture).
 void pf_ws_forget(hipStream_t s);
+int pf_ws_capture(hipStream_t s);
 // Per-device GEMM state (CU count, LDS limit, split-K workspace), set up by orc_init.
 int gemm_device_init(int device);
 void gemm_device_release();

@@ -735,17 +735,23 @@ __global__ __launch_bounds__(256) void k_pf_sum(QmvParams p, PfWork wk, const fl
 // its launches, and its stream first waits for the last use on any other
 // stream, so calls of any streams and threads take the workspace in turn.
 // Uses that follow each other on one of the library's own streams need no
-// event: the one a change of stream waits for is recorded then (or when the
-// stream is destroyed). An event after every use costs 4.4 us of GPU time
-// between two calls (3B blocks at 127 tokens: 22 of 222 us a layer). A stream
-// the library did not create may be destroyed behind its back, so its uses
-// are followed by an event at once.
+// event: it is recorded when another stream wants the workspace (which then
+// also waits for what the first stream has enqueued since), when a capture of
+// the stream begins (orc_graph_begin, under the lock: the event must not
+// become part of the capture) or when the stream is destroyed. An event after
+// every use costs 4.4 us of GPU time between two calls (3B blocks at 127
+// tokens: 22 of 222 us a layer). A stream the library did not create may be
+// destroyed behind its back, so its uses are followed by an event at once.
 // GEMM calls that need more than kPfWorkBytes go in token chunks.
 static std::mutex g_pf_mu;
 static uint8_t* g_pf_buf = nullptr;
 static hipEvent_t g_pf_ev = nullptr;
 static bool g_pf_ev_set = false;         // g_pf_ev follows the last use
 static hipStream_t g_pf_last = nullptr;  // or the last use is on this stream of the library
+
+static hipError_t pf_new_event(hipEvent_t* ev) {
+    return hipEventCreateWithFlags(ev, hipEventDisableTiming | hipEventDisableSystemFence);
+}
 
 void pf_release() {
     std::lock_guard<std::mutex> lk(g_pf_mu);
@@ -761,7 +767,7 @@ int pf_init() {
     pf_release();
     std::lock_guard<std::mutex> lk(g_pf_mu);
     ORC_HIP_CHECK(hipMalloc((void**)&g_pf_buf, kPfWorkBytes));
-    ORC_HIP_CHECK(hipEventCreateWithFlags(&g_pf_ev, hipEventDisableTiming | hipEventDisableSystemFence));
+    ORC_HIP_CHECK(pf_new_event(&g_pf_ev));
     return ORC_OK;
 }
 
@@ -777,8 +783,19 @@ int pf_ws_begin(hipStream_t s, uint8_t** buf) {
     if (!g_pf_buf) return set_error(ORC_E_NOINIT, "orc_init not called");
     if (g_pf_last != s) {
         if (g_pf_last) {
-            if (capturing(g_pf_last)) return kPfBusy;  // it cannot record an event now
+            // A capture of that stream that was begun through HIP itself: no
+            // event of it can be waited for, and it may begin between the
+            // question and the record. The event is then part of the capture:
+            // another one takes its place.
+            if (capturing(g_pf_last)) return kPfBusy;
             ORC_HIP_CHECK(hipEventRecord(g_pf_ev, g_pf_last));
+            if (capturing(g_pf_last)) {
+                hipEvent_t ev;
+                ORC_HIP_CHECK(pf_new_event(&ev));
+                (void)hipEventDestroy(g_pf_ev);
+                g_pf_ev = ev;
+                return kPfBusy;
+            }
             g_pf_last = nullptr;
             g_pf_ev_set = true;
         }
@@ -798,6 +815,17 @@ int pf_ws_end(hipStream_t s) {
     g_pf_last = nullptr;
     g_pf_ev_set = true;
     ORC_HIP_CHECK(hipEventRecord(g_pf_ev, s));
+    return ORC_OK;
+}
+
+int pf_ws_capture(hipStream_t s) {
+    std::lock_guard<std::mutex> lk(g_pf_mu);
+    if (g_pf_last == s && !capturing(s)) {
+        ORC_HIP_CHECK(hipEventRecord(g_pf_ev, s));
+        g_pf_last = nullptr;
+        g_pf_ev_set = true;
+    }
+    ORC_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     return ORC_OK;
 }
 

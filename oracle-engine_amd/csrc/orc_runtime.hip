@@ -179,8 +179,7 @@ extern "C" int orc_device_sync(void) {
 
 extern "C" int orc_graph_begin(orc_stream_t s) {
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
-    ORC_HIP_CHECK(hipStreamBeginCapture(resolve_stream(s), hipStreamCaptureModeThreadLocal));
-    return ORC_OK;
+    return pf_ws_capture(resolve_stream(s));
 }
 extern "C" int orc_graph_end(orc_stream_t s, orc_graph_t* out) {
     hipGraph_t g = nullptr;

@@ -1,0 +1,42 @@
+"""The library's host code without a GPU: streams, captures and the choice of
+kernels, over a pretended HIP runtime (tests/fake_hip.cpp) that writes the
+calls down. Everything here runs on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+import orc
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if not shutil.which("g++") or not os.path.exists(os.path.join(ROCM, "include", "hip", "hip_runtime_api.h")):
+        pytest.skip("no compiler or no HIP headers")
+    exe = str(tmp_path_factory.mktemp("fake") / "fake_hip")
+    lib = os.path.dirname(orc.HIP_LIB)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-rdynamic", "-I", os.path.join(ROCM, "include"),
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", exe, "-L", lib, "-lorc_hip",
+                    f"-Wl,-rpath,{lib}", "-Wl,--allow-shlib-undefined", "-ldl", "-lpthread"], check=True)
+
+    def run(*args):
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr
+        return r.stdout.splitlines()
+
+    return run
+
+
+@pytest.mark.parametrize("how", ["race", "race_hip"])
+def test_a_capture_begun_by_another_thread_pulls_no_stream_in(fake, how):
+    """A thread begins capturing the stream that used the prefill workspace
+    last, just as a call on another stream takes the workspace over."""
+    fake(how)
+
+
+def test_workspace_order_around_a_capture(fake):
+    fake("order")
