@@ -1017,7 +1017,7 @@ static int gemm_dispatch(QmvParams p, int type, hipStream_t s) {
     // the call's token count, never a chunk's, so chunking keeps results.
     const bool decode = p.n_tok == 1;
     if (decode && type == kMixK) return dispatch_mixed_decode(p, s);
-    if (pf_takes(type, p, s)) {
+    if (pf_takes(type, p)) {
         uint8_t* work = nullptr;
         int rc = pf_ws_begin(s, &work);
         if (!rc) {

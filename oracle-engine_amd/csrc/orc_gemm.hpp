@@ -71,18 +71,16 @@ int pf_init();
 void pf_release();
 // The workspace of the prefill kernels (one per device): 1024 tokens of 18944
 // split values (83 MB) with room for partial sums, or the split K and V of
-// 32 K positions of eight 128-wide kv heads. pf_ws_takes: whether `bytes` fit
-// and the stream is not being captured. pf_ws_begin locks it and orders the
-// stream behind its last use (kPfBusy: that was on a library stream whose
-// capture was begun through HIP itself instead of orc_graph_begin; the caller
-// takes a path without it); pf_ws_end ends the use and
-// unlocks. pf_ws_forget: a library stream is about to be destroyed.
+// 32 K positions of eight 128-wide kv heads. pf_ws_begin locks it and orders
+// the stream behind its last use; kPfBusy where the caller takes a path
+// without it: the stream is being captured, there is no workspace, or its last
+// use was on a library stream whose capture was begun through HIP itself
+// instead of orc_graph_begin. pf_ws_end ends the use and unlocks.
 constexpr size_t kPfWorkBytes = (size_t)256 << 20;
 constexpr int kPfBusy = 1;
-bool pf_ws_takes(hipStream_t s, size_t bytes);
 int pf_ws_begin(hipStream_t s, uint8_t** buf);
 int pf_ws_end(hipStream_t s);
-bool pf_takes(int type, const QmvParams& p, hipStream_t s);
+bool pf_takes(int type, const QmvParams& p);  // the shape; pf_ws_begin says the rest
 int pf_launch(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev, uint8_t* work);
 
 }  // namespace orc

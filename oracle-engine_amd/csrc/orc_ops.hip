@@ -1670,7 +1670,7 @@ extern "C" int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_
     bytes += 4.0 * n_tok * ((double)(n_heads + 2 * n_kv) * head_dim + (double)n_heads * head_dim);
     LaunchEv ev;
     uint8_t* work = nullptr;
-    int rc = pf_ws_takes(st, fa_bytes(head_dim, n_kv, pos_off + n_tok)) ? pf_ws_begin(st, &work) : kPfBusy;
+    int rc = fa_bytes(head_dim, n_kv, pos_off + n_tok) <= kPfWorkBytes ? pf_ws_begin(st, &work) : kPfBusy;
     if (rc && rc != kPfBusy) return rc;
     const bool tm = prof_arm(st, kProfAttnPf, n_tok, bytes, &ev.a, &ev.b);
     if (!rc) {

@@ -742,7 +742,9 @@ __global__ __launch_bounds__(256) void k_pf_sum(QmvParams p, PfWork wk, const fl
 // every use costs 4.4 us of GPU time between two calls (3B blocks at 127
 // tokens: 22 of 222 us a layer). A stream the library did not create may be
 // destroyed behind its back, so its uses are followed by an event at once.
-// GEMM calls that need more than kPfWorkBytes go in token chunks.
+// GEMM calls that need more than kPfWorkBytes go in token chunks. A device
+// without that much memory left has no workspace: calls take the kernels that
+// do without.
 static std::mutex g_pf_mu;
 static uint8_t* g_pf_buf = nullptr;
 static hipEvent_t g_pf_ev = nullptr;
@@ -766,8 +768,11 @@ void pf_release() {
 int pf_init() {
     pf_release();
     std::lock_guard<std::mutex> lk(g_pf_mu);
-    ORC_HIP_CHECK(hipMalloc((void**)&g_pf_buf, kPfWorkBytes));
     ORC_HIP_CHECK(pf_new_event(&g_pf_ev));
+    if (hipMalloc((void**)&g_pf_buf, kPfWorkBytes) != hipSuccess) {
+        g_pf_buf = nullptr;
+        (void)hipGetLastError();  // not the next launch's error
+    }
     return ORC_OK;
 }
 
@@ -776,11 +781,9 @@ static bool capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
 }
 
-bool pf_ws_takes(hipStream_t s, size_t bytes) { return g_pf_buf && bytes <= kPfWorkBytes && !capturing(s); }
-
 int pf_ws_begin(hipStream_t s, uint8_t** buf) {
     std::unique_lock<std::mutex> lk(g_pf_mu);
-    if (!g_pf_buf) return set_error(ORC_E_NOINIT, "orc_init not called");
+    if (!g_pf_buf || capturing(s)) return kPfBusy;
     if (g_pf_last != s) {
         if (g_pf_last) {
             // A capture of that stream that was begun through HIP itself: no
@@ -956,14 +959,14 @@ static int pf_split(const PfType& t, const PfSplit& sp, int ng, hipStream_t s, h
     return ORC_OK;
 }
 
-bool pf_takes(int type, const QmvParams& p, hipStream_t s) {
+bool pf_takes(int type, const QmvParams& p) {
     if (p.n_tok < kPfSplitMin || p.n_in % 32) return false;
     PfType t;
     if (type == kMixK) t = {2, true, true};
     else if (!pf_type(type, t)) return false;
     if (p.epi == ORC_EPI_SWIGLU && p.n_seg != 2) return false;
     PfWork w;
-    return pf_ws_takes(s, pf_layout(t, p.n_in, 4, nullptr, w));
+    return pf_layout(t, p.n_in, 4, nullptr, w) <= kPfWorkBytes;
 }
 
 int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& ev, uint8_t* buf) {

@@ -38,6 +38,7 @@ struct Wait {
 static std::recursive_mutex mu;
 static std::vector<Wait> waits;
 static std::vector<std::string> launches;
+static hipError_t last_error = hipSuccess;
 static size_t malloc_limit = ~(size_t)0;
 static std::function<void(Stream*)> on_query;  // called after the answer of hipStreamIsCapturing is settled
 static thread_local dim3 cfg_g, cfg_b;
@@ -83,11 +84,14 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
     return hipSuccess;
 }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    return last_error = hipSuccess, e;
+}
 const char* hipGetErrorString(hipError_t) { return "pretended error"; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { return *p = (void*)0x1000, hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) {
-    if (n > malloc_limit) return hipErrorOutOfMemory;
+    if (n > malloc_limit) return last_error = hipErrorOutOfMemory;
     return *p = std::malloc(16), hipSuccess;
 }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
@@ -194,12 +198,25 @@ static void capture_order() {
     CHECK(!orc_graph_end(a, &g) && !orc_stream_destroy(a) && !orc_stream_destroy(b));
 }
 
+// A device that has no 256 MB left: orc_init and every call work, on the
+// kernels that need no workspace.
+static void no_memory() {
+    malloc_limit = 100 << 20;
+    CHECK(!orc_init(0));
+    for (int type : {ORC_Q4_K, ORC_Q8_0, ORC_F16}) CHECK(!gemm(type, 300, 2048, 2048, nullptr));
+    const int H = 8, KV = 2, hd = 64, ld = (H + 2 * KV) * hd;
+    CHECK(!orc_attn_prefill(X, ld, 70, H, KV, hd, 50, X, X, X, 128, X, H * hd, nullptr));
+    CHECK(launches.size() >= 4);
+    for (const std::string& l : launches) CHECK(l.find("k_pf") == l.npos && l.find("k_kv_split") == l.npos);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc > 1);
     const std::string w = argv[1];
     if (w == "race") capture_race(true);
     else if (w == "race_hip") capture_race(false);
     else if (w == "order") capture_order();
+    else if (w == "no_memory") no_memory();
     else CHECK(!"a scenario");
     for (const std::string& l : launches) std::puts(l.c_str());
     return 0;

@@ -40,3 +40,7 @@ def test_a_capture_begun_by_another_thread_pulls_no_stream_in(fake, how):
 
 def test_workspace_order_around_a_capture(fake):
     fake("order")
+
+
+def test_init_without_memory_for_the_workspace(fake):
+    fake("no_memory")
