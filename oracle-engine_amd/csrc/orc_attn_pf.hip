@@ -18,6 +18,11 @@
 // products start from zero (the small ones apart for the scores, first for
 // P V), the blocks are added up in fp32 on the vector ALUs, and K and V are
 // stored negated in two of every four blocks.
+// Range: a block's probabilities are formed against its own row maximum
+// (rounded up to a power of two) and V against its own, so both halves of a
+// product hold their bits whatever the other blocks weigh; the running O and
+// sum keep their powers of two as integers, so adding a block up rounds
+// nothing but the sums themselves.
 #include "orc_gemm.hpp"
 #include "orc_attn_pf.hpp"
 
@@ -252,13 +257,18 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
         cq = ldexpf(1.4426950408889634f / sqrtf((float)HD), -eq);
     }
 
-    f16v o[DT];  // O^T: dims 32 dt + 8 (e / 4) + 4 h + e % 4 of the lane's row, times 2^14 2^-vr and the sign of `last`
+    // O^T: dims 32 dt + 8 (e / 4) + 4 h + e % 4 of the lane's row, times 2^(14 - u) and the sign of `last`
+    f16v o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-    float m = -INFINITY, l = 0.f;  // running maximum (log2 units), this lane's share of the sum
-    int vr = 120, last = 0;        // exponent of O's V scale (the smallest so far), sign it is held with
+    // whole numbers (log2 units), minus infinity before the first key: m the
+    // largest reference of a block, l this lane's share of the sum times 2^-m;
+    // u the power of two of O, um the largest a block asked for
+    float m = -INFINITY, l = 0.f, u = -INFINITY, um = -INFINITY;
+    int last = 0;
+    auto pow_of = [](float d) { return (int)fmaxf(d, -1000.f); };  // of a difference, which may be of infinities
 
     for (int bb = b0, it = 0; bb < b1; bb += KG, ++it) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies
@@ -292,24 +302,29 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int e = 0; e < 16; ++e) mb = fmaxf(mb, x[e]);
         mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-        const float mn = fmaxf(m, mb), mz = mn == -INFINITY ? 0.f : mn;  // no key yet: every p is 0
-        const float al = __builtin_amdgcn_exp2f(m - mz);
-        m = mn;
-        l *= al;
-        // P times V's power of two relative to O's and 2^14, as hi / lo halves
-        const int vn = min(vr, ve);
-        const float up = ldexpf(1.f, max(vn - ve, -100) + 14), ao = ldexpf(sg != last ? -al : al, max(vn - vr, -200));
-        vr = vn;
+        const float rf = ceilf(mb), rz = mb == -INFINITY ? 0.f : rf;  // no key yet: every p is 0
+        // O takes this block's power of two (its largest p near 1, times V's),
+        // at most 2^60 below the largest so far: what is smaller is below
+        // every rounding of the row
+        const float ub = rf - (float)ve;
+        um = fmaxf(um, ub);
+        const float un = fmaxf(ub, um - 60.f);
+        const float up = ldexpf(1.f, 14 + pow_of(ub - un)), ao = ldexpf(sg != last ? -1.f : 1.f, pow_of(u - un));
+        u = un;
         last = sg;
+        float lb = 0.f;
         u32x4 ph[2], pl[2];
 #pragma unroll
         for (int e = 0; e < 16; e += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(x[e] - mz), p1 = __builtin_amdgcn_exp2f(x[e + 1] - mz);
-            l += p0 + p1;
+            const float p0 = __builtin_amdgcn_exp2f(x[e] - rz), p1 = __builtin_amdgcn_exp2f(x[e + 1] - rz);
+            lb += p0 + p1;
             uint32_t lo;
             ph[e >> 3][(e & 7) >> 1] = split2(p0 * up, p1 * up, lo);
             pl[e >> 3][(e & 7) >> 1] = lo;
         }
+        const float mn = fmaxf(m, rf);
+        l = ldexpf(l, pow_of(m - mn)) + ldexpf(lb, pow_of(rf - mn));
+        m = mn;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
             h8v ah[2], alo[2];
@@ -334,11 +349,11 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
         }
     }
     l += __shfl_xor(l, 32, 64);
-    const float un = ldexpf(last ? -1.f : 1.f, -14 - vr);  // O to its own units
+    const int un = min(pow_of(u - m) - 14, 1000);  // O to the units of l
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[dt][e] *= un;
+        for (int e = 0; e < 16; ++e) o[dt][e] = ldexpf(last ? -o[dt][e] : o[dt][e], un);
 
     // merge of the key groups, in group order
     if constexpr (KG > 1) {

@@ -332,3 +332,71 @@ def test_narrow_matrices(dev, oracle, qt, nt, n_out, n_in):
     w, ty, W = _weights(dev, oracle, qt, n_out, n_in, rng)
     X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
     _check(_gemm(dev, ty, w, X, n_out), X, W)
+
+
+def _attn_case(dev, H, KVH, hd, sp, nt, S, K, V, qkv):
+    """orc_attn_prefill without rotation (angles 0), and the float64 result
+    over each row's own positions: (got, weights p [nt, H, S], float64 V)."""
+    ctx, ld = K.shape[1], (H + 2 * KVH) * hd
+    tab = np.zeros((ctx, hd // 2, 2), np.float32)
+    tab[..., 0] = 1
+    dq, dt, dK, dV = dev.upload(qkv), dev.upload(tab), dev.upload(K), dev.upload(V)
+    do = dev.alloc(nt * H * hd * 4)
+    dev.check(dev.L.orc_attn_prefill(dq.ptr, ld, nt, H, KVH, hd, sp, dt.ptr, dK.ptr, dV.ptr, ctx, do.ptr, H * hd, None))
+    got = do.read(np.float32).reshape(nt, H, hd)
+    x = qkv.astype(np.float64).reshape(nt, H + 2 * KVH, hd)
+    k64, v64 = K.astype(np.float64), V.astype(np.float64)
+    k64[:, sp:sp + nt], v64[:, sp:sp + nt] = x[:, H:H + KVH].transpose(1, 0, 2), x[:, H + KVH:].transpose(1, 0, 2)
+    p = np.zeros((nt, H, S))
+    for t in range(nt):
+        for h in range(H):
+            s = x[t, h] @ k64[h // (H // KVH), :sp + t + 1].T / np.sqrt(hd)
+            e = np.exp(s - s.max())
+            p[t, h, :sp + t + 1] = e / e.sum()
+    return got, p, v64
+
+
+def _scored(rng, H, KVH, hd, sp, nt, score, vscale):
+    """Inputs whose score of position j is score[j] (every query is the same
+    unit vector, every key that many times it) and whose V row j has the
+    magnitude vscale[j]."""
+    S = sp + nt
+    u = rng.normal(0, 1, hd)
+    u *= np.sqrt(np.sqrt(hd) / (u @ u))  # u . u / sqrt(hd) = 1
+    k = (score[:, None] * u).astype(np.float32)
+    qkv = np.zeros((nt, H + 2 * KVH, hd), np.float32)
+    qkv[:, :H] = u
+    K, V = np.zeros((KVH, S + 8, hd), np.float32), np.zeros((KVH, S + 8, hd), np.float32)
+    v = (rng.normal(0, 1, (KVH, S, hd)) * vscale[None, :, None]).astype(np.float32)
+    K[:, :sp], V[:, :sp] = k[:sp], v[:, :sp]
+    qkv[:, H:H + KVH], qkv[:, H + KVH:] = k[sp:, None], v[:, sp:].transpose(1, 0, 2)
+    return S, K, V, qkv.reshape(nt, -1)
+
+
+def _rows_within(got, p, v64, R, tol=6e-6):
+    """|error| <= tol times the row's sum of p_j max |v_j|: rounding in fp32 or
+    22 bits (2.4e-7 a product) of the two factors of every product, the
+    weights' own error (scores up to 40: 40 * 2^-24 = 2.4e-6) and the sums."""
+    v = np.repeat(v64, R, 0)
+    want, scale = np.einsum("ths,hsd->thd", p, v[:, :p.shape[2]]), np.einsum("ths,hs->th", p, np.abs(v[:, :p.shape[2]]).max(2))
+    err = np.abs(got - want).max(2) / scale
+    assert err.max() <= tol, (float(err.max()), np.unravel_index(err.argmax(), err.shape))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("big,drop", [(24, 40), (40, 60), (24, 17), (40, 28), (60, 80), (-40, 0)])
+def test_prefill_attention_v_ranges_over_blocks(dev, hd, big, drop):
+    """V of some blocks of 32 positions 2^big times the others', with scores
+    that give those positions exp(-drop) of the weight: a negligible large V, a
+    large V whose contribution is comparable, and a small V that carries all."""
+    print(f"[gpu] pf attention V range hd={hd} 2^{big} drop {drop}", flush=True)
+    rng = np.random.default_rng(hd + big + drop)
+    H, KVH, sp, nt = 4, 2, 300, 70
+    S = sp + nt
+    j = np.arange(S)
+    for blocks in ([0, 1], [4], [10], [0, 3, 6, 9]):
+        m = np.isin(j // 32, blocks)
+        score = np.where(m, -float(drop), rng.uniform(-2, 0, S))
+        vscale = np.where(m, 2.0 ** big, 1.0)
+        got, p, v64 = _attn_case(dev, H, KVH, hd, sp, nt, *_scored(rng, H, KVH, hd, sp, nt, score, vscale))
+        _rows_within(got, p, v64, H // KVH)
