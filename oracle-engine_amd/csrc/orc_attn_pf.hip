@@ -22,7 +22,11 @@
 // (rounded up to a power of two) and V against its own, so both halves of a
 // product hold their bits whatever the other blocks weigh; the running O and
 // sum keep their powers of two as integers, so adding a block up rounds
-// nothing but the sums themselves.
+// nothing but the sums themselves. Inside a block one power of two serves all
+// 32 positions: a block where some K or V row's largest value is below 2^-16
+// of the block's (its halves would keep fewer than 22 bits), or that holds an
+// infinity or NaN (which must not reach rows that do not see the position: 0
+// times infinity), is marked, and the waves take it in fp32 from the cache.
 #include "orc_gemm.hpp"
 #include "orc_attn_pf.hpp"
 
@@ -37,6 +41,7 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 typedef const __attribute__((address_space(1))) float* gfp;
 
 constexpr int kKB = 32;  // key positions per block
+constexpr int kPlain = 1024;  // an exponent's range is -128 .. 127
 template <int HD> constexpr int fa_block_bytes() { return HD * 256; }  // K and V fragments of a block
 
 // rotate-half of the pair (a, b) by (cos, sin): the rounding of every row rotation
@@ -64,8 +69,8 @@ __device__ __forceinline__ uint32_t split2(float a, float b, uint32_t& lo) {
 
 struct FaWork {
     uint8_t* frag;  // [kv head][block] fragments: K [dims 16 s][hi, lo], V [dims 32 dt][keys 16 s][hi, lo], 1 KB each
-    int* kexp;      // [kv head][block]: exponents of the stored K and V (value = stored 2^-exp)
-    int* vexp;
+    int* exps;      // [kv head][block]: exponents of the stored K (times 2^16) and V (value = stored 2^-exp), plus
+                    // kPlain where the block is taken in fp32
     int n_blk;
 };
 
@@ -79,6 +84,7 @@ __global__ __launch_bounds__(2 * HD) void k_kv_split(const float* qkv, int ldqkv
                                                      FaWork w) {
     constexpr int half = HD / 2, HS = HD / 32;
     __shared__ float red[2][2 * HD / 64];
+    __shared__ uint32_t rows[2 * HD / 64][5];
     const int blk = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
     const size_t kcol = (size_t)(n_heads + g) * HD, vcol = (size_t)(n_heads + n_kv + g) * HD;
     // every load first, without branches between them (positions past the end
@@ -122,13 +128,16 @@ __global__ __launch_bounds__(2 * HD) void k_kv_split(const float* qkv, int ldqkv
         if (pv >= start && pv < p_end) vc[((size_t)g * ctx + pv) * HD + d] = vv[i];
         if (pv >= p_end) vv[i] = 0.f;
     }
-    float mk = 0.f, mv = 0.f;
+    float mk = 0.f, mv = 0.f, rk;
+    bool odd = false;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {  // infinities and NaN set no scale
         const float a = fabsf(kv[i]), b = fabsf(vv[i]);
+        odd |= !(a <= 3.4028234e38f) || !(b <= 3.4028234e38f);
         mk = fmaxf(mk, a <= 3.4028234e38f ? a : 0.f);
         mv = fmaxf(mv, b <= 3.4028234e38f ? b : 0.f);
     }
+    rk = mk;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         mk = fmaxf(mk, __shfl_xor(mk, o, 64));
@@ -139,11 +148,26 @@ __global__ __launch_bounds__(2 * HD) void k_kv_split(const float* qkv, int ldqkv
     mk = red[0][0], mv = red[1][0];
 #pragma unroll
     for (int i = 1; i < 2 * HD / 64; ++i) mk = fmaxf(mk, red[0][i]), mv = fmaxf(mv, red[1][i]);
-    const int ek = up_exp(mk), ev = mv > 0.f ? up_exp(mv) : 120;  // a block of zeros never sets P V's scale
-    if (tid == 0) {
-        w.kexp[g * w.n_blk + blk] = ek;
-        w.vexp[g * w.n_blk + blk] = ev;
+    // positions with a value that is not zero, and with one of at least 2^-16
+    // of the largest, as bits: K's two rows of lanes hold the same positions,
+    // V's lanes hold 16 positions each
+    {
+        const unsigned long long n2 = __ballot(rk > 0.f), g2 = __ballot(rk >= mk * 0x1p-16f && rk > 0.f);
+        uint32_t nv = 0, gv = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float a = fabsf(vv[i]);
+            nv |= __ballot(a > 0.f) ? 1u << i : 0u;
+            gv |= __ballot(a >= mv * 0x1p-16f && a > 0.f) ? 1u << i : 0u;
+        }
+        const bool any_odd = __ballot(odd) != 0;
+        if ((tid & 63) == 0) {
+            uint32_t* d = rows[tid >> 6];
+            d[0] = (uint32_t)n2 | (uint32_t)(n2 >> 32), d[1] = (uint32_t)g2 | (uint32_t)(g2 >> 32);
+            d[2] = nv << (16 * s2), d[3] = gv << (16 * s2), d[4] = any_odd;
+        }
     }
+    const int ek = up_exp(mk), ev = mv > 0.f ? up_exp(mv) : 120;  // a block of zeros never sets P V's scale
     const float sg = sign_of(blk) ? -1.f : 1.f, uk = ldexpf(sg, ek), uv = ldexpf(sg, ev);
     uint8_t* f = w.frag + ((size_t)g * w.n_blk + blk) * fa_block_bytes<HD>();
 #pragma unroll
@@ -169,6 +193,15 @@ __global__ __launch_bounds__(2 * HD) void k_kv_split(const float* qkv, int ldqkv
         *(u32x4*)o = hi;
         *(u32x4*)(o + 1024) = lo;
     }
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t d[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2 * HD / 64; ++i)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) d[k] |= rows[i][k];
+        w.exps[g * w.n_blk + blk] = ek * 65536 + ev + (d[0] != d[1] || d[2] != d[3] || d[4] ? kPlain : 0);
+    }
 }
 
 // RT row tiles of 32 x KG key groups: wave (rt, kg) takes its 32 rows through
@@ -179,8 +212,8 @@ __global__ __launch_bounds__(2 * HD) void k_kv_split(const float* qkv, int ldqkv
 // the next KG while these multiply.
 template <int HD, int RT, int KG>
 __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_fa(
-    const float* qkv, int ldqkv, int n_tok, int n_heads, int n_kv, int start, const float2* rope, FaWork w, float* out,
-    int ldo, float* part, int nz) {
+    const float* qkv, int ldqkv, int n_tok, int n_heads, int n_kv, int start, const float2* rope, const float* kc,
+    const float* vc, int ctx, FaWork w, float* out, int ldo, float* part, int nz) {
     constexpr int half = HD / 2, KS = HD / 16, DT = HD / 32, NW = RT * KG, BB = fa_block_bytes<HD>(), NF = KG * BB / 1024 / NW;
     static_assert(KG * BB / 1024 % NW == 0, "whole fragments");
     extern __shared__ __attribute__((aligned(16))) uint8_t sm[];  // [2][KG][block]
@@ -196,11 +229,10 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
     const int per = (all + nz * KG - 1) / (nz * KG) * KG, b0 = min(all, z * per), b1 = min(all, b0 + per);  // this range's
     const int r = rt * 32 + n, rc = r < NR ? r : 0, ti = rc / R, hd = rc - ti * R, pt = start + t0 + ti;
     const uint8_t* fr = w.frag + (size_t)g * w.n_blk * BB;
-    const int* kx = w.kexp + g * w.n_blk;
-    const int* vx = w.vexp + g * w.n_blk;
+    const int* ex = w.exps + g * w.n_blk;
 
     auto copy = [&](int blk, int buf) {  // blocks blk .. blk + KG - 1 (those below b1)
-#pragma unroll
+#pragma unroll 8
         for (int i = 0; i < NF; ++i) {
             const int f = wave + i * NW, j = f / (BB / 1024);
             if (blk + j < b1)
@@ -209,6 +241,9 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
                     (__attribute__((address_space(3))) void*)(sm + (buf * KG * BB + f * 1024)), 16, 0, 0);
         }
     };
+    // this wave's exponents a round ahead, in front of the copies: a wait for
+    // them is then no wait for the copies that follow
+    int xn = b0 < b1 ? ex[min(b0 + kg, b1 - 1)] : 0;
     if (b0 < b1) copy(b0, 0);
 
     // the row's rotated query as B operands: dims 16 s + 8 h + 0 .. 7
@@ -270,27 +305,37 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
     int last = 0;
     auto pow_of = [](float d) { return (int)fmaxf(d, -1000.f); };  // of a difference, which may be of infinities
 
+    bool any = false;  // a marked block was left out
     for (int bb = b0, it = 0; bb < b1; bb += KG, ++it) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies
         __syncthreads();  // every wave's; the other buffer's readers are done
+        const int b = bb + kg, xb = __builtin_amdgcn_readfirstlane(xn), ve = (int16_t)xb, ke = (xb - ve) >> 16;
+        xn = ex[min(b + KG, b1 - 1)];
         if (bb + KG < b1) copy(bb + KG, (it + 1) & 1);
-        const int b = bb + kg;
         if (b >= b1) continue;  // uniform over the wave
         const uint8_t* kf = sm + ((it & 1) * KG + kg) * BB + lane * 16;
         const uint8_t* vf = kf + KS * 2048;
         f16v sh, sl;
 #pragma unroll
         for (int e = 0; e < 16; ++e) sh[e] = sl[e] = 0.f;
+        h8v ah[2], al[2];  // the next step's fragments are read in front of a step's products
+        auto read = [&](int s) { ah[s & 1] = *(const h8v*)(kf + s * 2048), al[s & 1] = *(const h8v*)(kf + s * 2048 + 1024); };
+        read(0);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            const h8v ah = *(const h8v*)(kf + s * 2048), al = *(const h8v*)(kf + s * 2048 + 1024);
-            sh = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qh[s], sh, 0, 0, 0);
-            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qh[s], sl, 0, 0, 0);
-            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ql[s], sl, 0, 0, 0);
+            if (s + 1 < KS) read(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            sh = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s & 1], qh[s], sh, 0, 0, 0);
+            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s & 1], qh[s], sl, 0, 0, 0);
+            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s & 1], ql[s], sl, 0, 0, 0);
+        }
+        if (ve >= kPlain / 2) {
+            any = true;
+            continue;
         }
         // scores in log2 units; keys 8 (e / 4) + 4 h + e % 4 of the block
-        const int sg = sign_of(b), ve = vx[b];
-        const float c = ldexpf(sg ? -cq : cq, -kx[b]);
+        const int sg = sign_of(b);
+        const float c = ldexpf(sg ? -cq : cq, -ke);
         float x[16], mb = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 16; ++e) x[e] = (sh[e] + sl[e]) * c;
@@ -327,25 +372,110 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
         m = mn;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            h8v ah[2], alo[2];
+            h8v vh[2], vl[2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                ah[s] = *(const h8v*)(vf + (dt * 2 + s) * 2048);
-                alo[s] = *(const h8v*)(vf + (dt * 2 + s) * 2048 + 1024);
+                vh[s] = *(const h8v*)(vf + (dt * 2 + s) * 2048);
+                vl[s] = *(const h8v*)(vf + (dt * 2 + s) * 2048 + 1024);
             }
             f16v y;
 #pragma unroll
             for (int e = 0; e < 16; ++e) y[e] = 0.f;
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(alo[s], __builtin_bit_cast(h8v, ph[s]), y, 0, 0, 0);
-                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], __builtin_bit_cast(h8v, pl[s]), y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[s], __builtin_bit_cast(h8v, ph[s]), y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], __builtin_bit_cast(h8v, pl[s]), y, 0, 0, 0);
             }
 #pragma unroll
             for (int s = 0; s < 2; ++s)
-                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], __builtin_bit_cast(h8v, ph[s]), y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], __builtin_bit_cast(h8v, ph[s]), y, 0, 0, 0);
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[dt][e] = __builtin_fmaf(ao, o[dt][e], y[e]);
+        }
+    }
+    // The marked blocks, in fp32 from the cache, value after value in every
+    // lane: positions a row does not see are left out, and every position is
+    // added at its own power of two. After the others, where the registers of
+    // the split query are free.
+    for (int b = b0 + kg; any && b < b1; b += KG) {
+        if ((int16_t)__builtin_amdgcn_readfirstlane(ex[b]) < kPlain / 2) continue;
+        int rp = rc;
+        asm volatile("" : "+v"(rp));  // the row's addresses are formed here, not held through the loop above
+        const int tp = t0 + rp / R;
+        const float* q = qkv + (size_t)tp * ldqkv + (size_t)(g * R + rp % R) * HD;
+        const float2* cs = rope + (size_t)(start + tp) * half;
+        const size_t row0 = (size_t)g * ctx;
+        const int lastp = start + n_tok - 1;
+        float x[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] = 0.f;
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {  // positions 8 i + 4 h + 0 .. 3
+            float s4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int d = 0; d < half; ++d) {
+                const float2 c = cs[d];
+                const float qa = rot_lo(q[d], q[half + d], c), qb = rot_hi(q[d], q[half + d], c);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float* k = kc + (row0 + min(b * kKB + 8 * i + 4 * h + j, lastp)) * HD + d;
+                    s4[j] = __builtin_fmaf(qa, k[0], __builtin_fmaf(qb, k[half], s4[j]));
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 12; ++e) x[e] = x[e + 4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                x[12 + j] = b * kKB + 8 * i + 4 * h + j > pt ? -INFINITY : s4[j] * (1.4426950408889634f / sqrtf((float)HD));
+        }
+        float mb = -INFINITY, lb = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mb = fmaxf(mb, x[e]);
+        mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+        const float rf = ceilf(mb), rz = mb == -INFINITY ? 0.f : rf, mn = fmaxf(m, rf);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lb += __builtin_amdgcn_exp2f(x[e] - rz);
+        l = ldexpf(l, pow_of(m - mn)) + ldexpf(lb, pow_of(rf - mn));
+        m = mn;
+#pragma unroll 1
+        for (int i = 0; i < 16; ++i) {
+            const float own = x[0], other = __shfl_xor(own, 32, 64);
+#pragma unroll
+            for (int e = 0; e < 15; ++e) x[e] = x[e + 1];
+#pragma unroll 1
+            for (int hh = 0; hh < 2; ++hh) {
+                const int key = b * kKB + 8 * (i >> 2) + 4 * hh + (i & 3);
+                if (key > pt) continue;
+                const float xs = hh == h ? own : other, rs = xs == -INFINITY ? 0.f : ceilf(xs);
+                const float ps = __builtin_amdgcn_exp2f(xs - rs);
+                const float* vp = vc + (row0 + key) * HD + 4 * h;  // read twice: the registers are full
+                float mv = 0.f;
+#pragma unroll 1
+                for (int d = 0; d < HD; d += 8) {
+                    const float4 a = *(const float4*)(vp + d);
+                    const float v[4] = {fabsf(a.x), fabsf(a.y), fabsf(a.z), fabsf(a.w)};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) mv = fmaxf(mv, v[k] <= 3.4028234e38f ? v[k] : 0.f);
+                }
+                const float ub = mv > 0.f && xs > -INFINITY ? rs - (float)up_exp(mv) : -INFINITY;
+                um = fmaxf(um, ub);
+                const float un = fmaxf(ub, um - 60.f);
+                const int eo = pow_of(u - un), ev = min(pow_of(rs + 14.f - un), 1000);
+                u = un;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4) {
+                        const float4 a = *(const float4*)(vp + 32 * dt + 8 * q4);
+                        const float v[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const int e = 4 * q4 + k;
+                            o[dt][e] = __builtin_fmaf(last ? -ps : ps, ldexpf(v[k], ev), ldexpf(o[dt][e], eo));
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
         }
     }
     l += __shfl_xor(l, 32, 64);
@@ -434,10 +564,10 @@ static void fa_go(const FaArgs& a, const FaWork& w, int nz, float* part, hipEven
     const dim3 grid((a.n_tok + TB - 1) / TB * a.n_kv, nz);
     if (stop && nz == 1)
         hipExtLaunchKernelGGL((k_attn_fa<HD, RT, KG>), grid, dim3(64 * RT * KG), (fa_lds<HD, RT, KG>()), a.s, nullptr, stop, 0,
-                              a.qkv, a.ldqkv, a.n_tok, a.n_heads, a.n_kv, a.start, a.rope, w, a.out, a.ldo, part, nz);
+                              a.qkv, a.ldqkv, a.n_tok, a.n_heads, a.n_kv, a.start, a.rope, a.kc, a.vc, a.ctx, w, a.out, a.ldo, part, nz);
     else
         hipLaunchKernelGGL((k_attn_fa<HD, RT, KG>), grid, dim3(64 * RT * KG), (fa_lds<HD, RT, KG>()), a.s, a.qkv, a.ldqkv,
-                           a.n_tok, a.n_heads, a.n_kv, a.start, a.rope, w, a.out, a.ldo, part, nz);
+                           a.n_tok, a.n_heads, a.n_kv, a.start, a.rope, a.kc, a.vc, a.ctx, w, a.out, a.ldo, part, nz);
     if (nz > 1) {
         const dim3 g2(a.n_tok, a.n_heads);
         if (stop)
@@ -454,8 +584,7 @@ template <int HD> static int fa_run(const FaArgs& a, uint8_t* buf, size_t cap, h
     w.n_blk = (p_end + kKB - 1) / kKB;
     const size_t frag = (size_t)a.n_kv * w.n_blk * fa_block_bytes<HD>();
     w.frag = buf;
-    w.kexp = (int*)(buf + frag);
-    w.vexp = w.kexp + (size_t)a.n_kv * w.n_blk;
+    w.exps = (int*)(buf + frag);
     const size_t used = fa_bytes(HD, a.n_kv, p_end);
     const dim3 grid(w.n_blk, a.n_kv);
     if (start)
@@ -481,7 +610,7 @@ template <int HD> static int fa_run(const FaArgs& a, uint8_t* buf, size_t cap, h
 
 size_t fa_bytes(int hd, int n_kv, int p_end) {
     const size_t n = (size_t)n_kv * ((p_end + kKB - 1) / kKB);
-    return (n * (hd * 256 + 2 * sizeof(int)) + 255) / 256 * 256;
+    return (n * (hd * 256 + sizeof(int)) + 255) / 256 * 256;
 }
 
 int fa_launch(int head_dim, const FaArgs& a, uint8_t* work, hipEvent_t start, hipEvent_t stop) {

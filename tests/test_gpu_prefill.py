@@ -351,8 +351,9 @@ def _attn_case(dev, H, KVH, hd, sp, nt, S, K, V, qkv):
     for t in range(nt):
         for h in range(H):
             s = x[t, h] @ k64[h // (H // KVH), :sp + t + 1].T / np.sqrt(hd)
-            e = np.exp(s - s.max())
-            p[t, h, :sp + t + 1] = e / e.sum()
+            with np.errstate(invalid="ignore"):  # a row that sees an infinity
+                e = np.exp(s - s.max())
+                p[t, h, :sp + t + 1] = e / e.sum()
     return got, p, v64
 
 
@@ -400,3 +401,62 @@ def test_prefill_attention_v_ranges_over_blocks(dev, hd, big, drop):
         vscale = np.where(m, 2.0 ** big, 1.0)
         got, p, v64 = _attn_case(dev, H, KVH, hd, sp, nt, *_scored(rng, H, KVH, hd, sp, nt, score, vscale))
         _rows_within(got, p, v64, H // KVH)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("what", ["v", "v_comparable", "v_later", "k_later", "k_low"])
+def test_prefill_attention_ranges_inside_a_block(dev, hd, what):
+    """V (or K) rows 2^20 to 2^50 apart inside a block of 32 positions, the
+    large ones of little weight, of comparable weight, or not seen by the
+    earlier tokens of the pass."""
+    print(f"[gpu] pf attention range in a block hd={hd} {what}", flush=True)
+    rng = np.random.default_rng(hd + len(what))
+    H, KVH, sp, nt = 6, 2, 77, 90
+    S = sp + nt
+    j = np.arange(S)
+    score, vscale = rng.uniform(-2, 0, S), np.ones(S)
+    big = (j % 5 == 2) & (j > 20)
+    if what == "v":
+        score[big], vscale[big] = -60.0, 2.0 ** rng.integers(20, 50, big.sum())
+    elif what == "v_comparable":
+        b = rng.integers(20, 50, big.sum())
+        score[big], vscale[big] = -b * np.log(2.0) + rng.uniform(-2, 2, big.sum()), 2.0 ** b
+    elif what == "v_later":
+        vscale[j >= sp + 50] = 2.0 ** 40
+    elif what == "k_later":
+        score[j >= sp + 50] = 2.0 ** 30 * rng.choice([-1, 1], nt - 50)
+    else:
+        score[big] = -2.0 ** 30
+    got, p, v64 = _attn_case(dev, H, KVH, hd, sp, nt, *_scored(rng, H, KVH, hd, sp, nt, score, vscale))
+    n = 50 if what == "k_later" else nt  # (scores near 2^30 tie in fp32: tokens that see them are not compared)
+    _rows_within(got[:n], p[:n], v64, H // KVH)
+
+
+@pytest.mark.parametrize("H,KVH,hd,nt", [(4, 4, 64, 150), (8, 2, 64, 40), (4, 4, 128, 150), (14, 2, 128, 70)])
+def test_prefill_attention_infinities_reach_no_earlier_token(dev, H, KVH, hd, nt):
+    """A V or K row with an infinity or NaN changes no token before its
+    position; later tokens have it in the dimensions it is in."""
+    print(f"[gpu] pf attention infinities H={H} KVH={KVH} hd={hd} nt={nt}", flush=True)
+    rng = np.random.default_rng(H + hd)
+    sp = 45
+    S, K, V, qkv = _scored(rng, H, KVH, hd, sp, nt, rng.uniform(-2, 0, sp + nt), np.ones(sp + nt))
+    qkv = qkv.reshape(nt, H + 2 * KVH, hd)
+    at = nt - 7
+    want, p, v64 = _attn_case(dev, H, KVH, hd, sp, nt, S, K, V, qkv.reshape(nt, -1))
+    for bad in (np.inf, -np.inf, np.nan):
+        q = qkv.copy()
+        q[at, H + KVH:, 3] = bad
+        got, _, _ = _attn_case(dev, H, KVH, hd, sp, nt, S, K, V, q.reshape(nt, -1))
+        _rows_within(got[:at], p[:at], v64, H // KVH)
+        assert np.array_equal(got[at:, :, 3], np.full((nt - at, H), bad, np.float32), equal_nan=True)
+        rest = np.r_[0:3, 4:hd]
+        assert np.allclose(got[at:][:, :, rest], want[at:][:, :, rest], rtol=0, atol=2e-5)
+        q = qkv.copy()
+        q[at, H:H + KVH, 3] = bad
+        got, _, _ = _attn_case(dev, H, KVH, hd, sp, nt, S, K, V, q.reshape(nt, -1))
+        _rows_within(got[:at], p[:at], v64, H // KVH)
+    # in the cache before the pass: every token has it
+    V2 = V.copy()
+    V2[:, 40, 5] = np.inf
+    got, _, _ = _attn_case(dev, H, KVH, hd, sp, nt, S, K, V2, qkv.reshape(nt, -1))
+    assert np.isposinf(got[:, :, 5]).all() and np.isfinite(np.delete(got, 5, 2)).all()
