@@ -1011,13 +1011,42 @@ static int dispatch_mixed_decode(const QmvParams& p, hipStream_t s) {
     return ORC_OK;
 }
 
+// Whether the verify kernels take a short prompt call over a small K-quant or
+// dense matrix in less time than the two or three launches of the prefill
+// kernels, by the rounds of workgroups over the CUs: a K-quant launch is 2 us
+// and 6.4 + n_in / 1024 a round (9 + n_in / 1024 for mixed types, 1.4 times
+// that for SwiGLU pairs; a remainder of tokens is a second launch), a dense one
+// 4.1 + n_in / 1900 and 2.6 + n_in / 2900. Measured (us, verify against prefill
+// kernels): 2048 x 2048 Q6_K at 32 tokens 11.0 and 16.7, at 48 19.7 and 17.2;
+// 896 x 1024 Q4_K at 64 10.3 and 13.3, at 128 18.3 and 13.8; 512 x 512 Q6_K at
+// 128 9.0 and 13.7; 1024 + 256 + 256 mixed rows x 1024 at 32 12.7 and 23.8, at
+// 64 22.8 and 24.1; 64 x 1024 F16 at 40 7.0 and 11.8, at 48 15.0 and 11.7. Q8_0 and Q4_0 matrices of at most 256 rows would gain as
+// dense ones do, but their vector kernels make a NaN of an infinite activation
+// where the prefill kernels keep the infinity: they stay.
+static bool verify_faster(int type, const QmvParams& p) {
+    const bool kq = mmq_type(type), pair = p.epi == ORC_EPI_SWIGLU;
+    if (kq ? p.n_tok >= kPfMinTok : (type != ORC_F16 && type != ORC_BF16) || p.n_tok > 100 || p.n_rows > 512 || pair)
+        return false;
+    const int nt = kq ? mmq_max_tokens(type, p) : max_tokens(type, p.n_in);
+    if (nt < 1) return false;
+    const int whole = std::max(1, p.n_tok / nt), rem = p.n_tok >= nt ? p.n_tok % nt : 0;
+    const long rows = pair ? p.rows[0] : p.n_rows, groups = kq ? (rows + 15) / 16 : (rows + 1) / 2;
+    auto rounds = [&](int blocks) { return (double)((blocks * groups + g_n_cu - 1) / g_n_cu); };
+    const double k = p.n_in / 1024.0, r = rounds(whole);
+    if (!kq && r > 1 && p.n_in > 3072) return false;  // longer than the line above says
+    double us;
+    if (kq) us = 2 + r * ((type == kMixK ? 9.0 : 6.4) + k) * (pair ? 1.4 : 1) + (rem ? rounds(1) * (3.3 + 0.25 * rem) : 0);
+    else us = 4.1 + 0.55 * k + r * (2.6 + 0.35 * k) + (rem ? rounds(1) * (2.7 + rem * (0.54 + 0.18 * k)) : 0);
+    return us + (p.norm_w ? 1.0 : 0.0) < 0.96 * pf_estimate(type, p);
+}
+
 static int gemm_dispatch(QmvParams p, int type, hipStream_t s) {
     // a one-token call (decode) runs on the vector ALUs for every type; the
     // K-quants take the matrix cores from two tokens up. The choice follows
     // the call's token count, never a chunk's, so chunking keeps results.
     const bool decode = p.n_tok == 1;
     if (decode && type == kMixK) return dispatch_mixed_decode(p, s);
-    if (pf_takes(type, p)) {
+    if (pf_takes(type, p) && !verify_faster(type, p)) {
         uint8_t* work = nullptr;
         int rc = pf_ws_begin(s, &work);
         if (!rc) {

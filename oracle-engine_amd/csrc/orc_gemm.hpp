@@ -65,7 +65,9 @@ int mmq_prefill_launch(int type, const QmvParams& p, hipStream_t s, const Launch
 // kernels' 16-token block and its remainder do on the smallest K-quant matrix
 // (3072 x 3072 Q4_K: 21 us either way; at 20 tokens 21 against 18, at 32 21
 // against 27); every larger or vector-kernel matrix gains earlier (7B gate+up
-// Q6_K at 20 tokens 70 against 158 us). Verify passes stay below it.
+// Q6_K at 20 tokens 70 against 158 us). Verify passes stay below it, and small
+// K-quant and dense matrices stay with the verify kernels for more tokens
+// (verify_faster, orc_gemm.hip).
 constexpr int kPfSplitMin = 24;
 int pf_init();
 void pf_release();
@@ -81,6 +83,7 @@ constexpr int kPfBusy = 1;
 int pf_ws_begin(hipStream_t s, uint8_t** buf);
 int pf_ws_end(hipStream_t s);
 bool pf_takes(int type, const QmvParams& p);  // the shape; pf_ws_begin says the rest
+double pf_estimate(int type, const QmvParams& p);  // microseconds of a small call
 int pf_launch(int type, const QmvParams& p, hipStream_t s, const LaunchEvents& ev, uint8_t* work);
 
 }  // namespace orc

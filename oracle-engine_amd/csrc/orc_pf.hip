@@ -938,6 +938,34 @@ static PfPlan pf_plan(int type, const QmvParams& p, int supers) {
     return r;
 }
 
+// Microseconds of a launch pair by its longest chain: per superblock of a range
+// 2.7 (4.8 for rows whose loads wait for each other), 3 more with 64-token
+// tiles, per round of workgroups 3.5, the sum of the ranges 1.6 + 0.15 each; the
+// norm 1, SwiGLU 1.5, the launches of a second weight type 6.
+// Within 5% (rms) of the measured times of 61 matrices of 64 to 8192 rows and
+// 256 to 8192 values at 24 to 255 tokens, up to about 25 us; above that the
+// products count, and it is far too low.
+double pf_estimate(int type, const QmvParams& p) {
+    const int supers = (p.n_in + kSuper - 1) / kSuper;
+    double us = 3.5 + (p.norm_w ? 1.0 : 0.0) + (p.epi == ORC_EPI_SWIGLU ? 1.5 : 0.0);
+    for (int i0 = 0; i0 < p.n_seg;) {
+        QmvParams q = p;
+        int i1 = i0;
+        q.n_rows = 0;
+        for (; i1 < p.n_seg && p.seg_type[i1] == p.seg_type[i0]; ++i1) q.n_rows += p.rows[i1];
+        const int ty = p.seg_type[i0];
+        const PfPlan r = pf_plan(ty, q, supers);
+        const int bt = r.shape == 0 ? 128 : r.shape == 1 ? 64 : 32;
+        const int rows = p.epi == ORC_EPI_SWIGLU ? 2 * p.rows[0] : q.n_rows;
+        const long wgs = (long)((rows + 127) / 128) * ((p.n_tok + bt - 1) / bt) * r.nz;
+        const bool serial = ty == ORC_Q8_0 || ty == ORC_Q8_0_X8 || ty == ORC_Q4_0;
+        us += (i0 ? 6.0 : 0.0) + 3.5 * ((wgs + g_n_cu - 1) / g_n_cu) + ((serial ? 4.8 : 2.7) + (r.shape == 2 ? 0 : 3)) * ((supers + r.nz - 1) / r.nz);
+        if (r.nz > 1) us += 1.6 + 0.15 * r.nz;
+        i0 = i1;
+    }
+    return us;
+}
+
 template <int QT>
 static int pf_run(const QmvParams& p, const PfWork& w, const PfPlan& r, float* part, hipStream_t s, hipEvent_t stop) {
     if constexpr (QT != ORC_BF16)

@@ -210,6 +210,17 @@ static void no_memory() {
     for (const std::string& l : launches) CHECK(l.find("k_pf") == l.npos && l.find("k_kv_split") == l.npos);
 }
 
+// gemm type n_tok n_out n_in | attn heads kv head_dim n_tok pos: the call's launches
+static void route(int argc, char** argv) {
+    CHECK(argc == 6 + (argv[1][0] == 'a'));
+    int v[5];
+    for (int i = 2; i < argc; ++i) v[i - 2] = std::atoi(argv[i]);
+    CHECK(!orc_init(0));
+    if (argv[1][0] == 'g') CHECK(!gemm(v[0], v[1], v[2], v[3], nullptr));
+    else
+        CHECK(!orc_attn_prefill(X, (v[0] + 2 * v[1]) * v[2], v[3], v[0], v[1], v[2], v[4], X, X, X, v[4] + v[3], X, v[0] * v[2], nullptr));
+}
+
 int main(int argc, char** argv) {
     CHECK(argc > 1);
     const std::string w = argv[1];
@@ -217,6 +228,7 @@ int main(int argc, char** argv) {
     else if (w == "race_hip") capture_race(false);
     else if (w == "order") capture_order();
     else if (w == "no_memory") no_memory();
+    else if (w == "gemm" || w == "attn") route(argc, argv);
     else CHECK(!"a scenario");
     for (const std::string& l : launches) std::puts(l.c_str());
     return 0;

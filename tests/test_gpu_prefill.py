@@ -79,11 +79,14 @@ def test_against_float64(dev, oracle, qt, nt, n_out, n_in):
 def test_epilogues(dev, oracle, qt, nt, n_in):
     """RMSNorm prologue with bias into three segments, SwiGLU pairs (rows not a
     multiple of 16) and residual accumulation, in float64."""
+    _epilogues(dev, oracle, qt, nt, n_in, (45, 33, 50))
+
+
+def _epilogues(dev, oracle, qt, nt, n_in, rows):
     import orc
 
-    print(f"[gpu] pf epilogues type={qt} nt={nt} n_in={n_in}", flush=True)
+    print(f"[gpu] pf epilogues type={qt} nt={nt} n_in={n_in} rows={rows}", flush=True)
     rng = np.random.default_rng(7 * nt)
-    rows = (45, 33, 50)
     ws = [_weights(dev, oracle, qt, r, n_in, rng) for r in rows]
     X = rng.normal(0, 3, (nt, n_in)).astype(np.float32)
     g = rng.uniform(0.5, 1.5, n_in).astype(np.float32)
@@ -105,7 +108,7 @@ def test_epilogues(dev, oracle, qt, nt, n_in):
         want = dot[i] + (bias if i == 1 else 0)
         assert np.all(np.abs(got[:, offs[i]:offs[i + 1]] - want) <= 2e-6 * scale[i] + 3e-7 * np.abs(want)), i
     # SwiGLU over the first rows of two segments
-    ff = 33
+    ff = rows[1]
     segs = (orc.Seg * 2)(orc.Seg(ws[0][0].ptr, ff, dy.ptr, None), orc.Seg(ws[1][0].ptr, ff, dy.ptr, None))
     dev.check(dev.L.orc_gemm_fused(qt, segs, 2, nt, n_in, dx.ptr, n_in, ff, dg.ptr, C.c_float(1e-5), orc.EPI_SWIGLU,
                                    None))
@@ -127,10 +130,14 @@ def test_epilogues(dev, oracle, qt, nt, n_in):
 
 def test_mixed_segments(dev, oracle):
     """Q4_K and Q6_K segments of one call (a Q4_K_M layer's Q|K|V) share one split."""
+    _mixed(dev, oracle, 1024, (96, 32, 64), 70)
+
+
+def _mixed(dev, oracle, n_in, rows, nt):
     import orc
 
     rng = np.random.default_rng(5)
-    n_in, rows, types, nt = 1024, (96, 32, 64), (ol.Q4_K, ol.Q6_K, ol.Q6_K), 70
+    types = (ol.Q4_K, ol.Q6_K, ol.Q6_K)
     ws = [_weights(dev, oracle, t, r, n_in, rng) for t, r in zip(types, rows)]
     X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
     dx, dy = dev.upload(X), dev.alloc(nt * sum(rows) * 4)
@@ -142,6 +149,26 @@ def test_mixed_segments(dev, oracle):
     got = dy.read(np.float32).reshape(nt, -1)
     for i in range(3):
         _check(got[:, offs[i]:offs[i + 1]], X, ws[i][2])
+
+
+# K-quants at sizes that go to the prefill kernels (smaller matrices stay with
+# the verify kernels for these token counts): the tile edges of CASES
+K_CASES = [(ol.Q4_K, 24, 8223, 256), (ol.Q4_K, 33, 4226, 2304), (ol.Q6_K, 32, 8225, 256), (ol.Q6_K, 65, 1151, 4352),
+           (ol.Q4_K, 130, 1090, 1280), (ol.Q6_K, 257, 65, 512)]
+
+
+@pytest.mark.parametrize("qt,nt,n_out,n_in", K_CASES)
+def test_k_quants_against_float64(dev, oracle, qt, nt, n_out, n_in):
+    test_against_float64(dev, oracle, qt, nt, n_out, n_in)
+
+
+@pytest.mark.parametrize("qt,nt,n_in,rows", [(ol.Q4_K, 50, 512, (4173, 4161, 50)), (ol.Q6_K, 140, 2304, (1061, 1041, 33))])
+def test_k_quant_epilogues(dev, oracle, qt, nt, n_in, rows):
+    _epilogues(dev, oracle, qt, nt, n_in, rows)
+
+
+def test_mixed_segments_at_prefill_sizes(dev, oracle):
+    _mixed(dev, oracle, 1024, (2080, 1040, 1056), 70)
 
 
 @pytest.mark.parametrize("qt", [ol.Q8_0, ol.F16, ol.BF16])

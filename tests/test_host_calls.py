@@ -44,3 +44,25 @@ def test_workspace_order_around_a_capture(fake):
 
 def test_init_without_memory_for_the_workspace(fake):
     fake("no_memory")
+
+
+Q4_K, Q6_K, Q8_0, Q4_0, F16 = 12, 14, 8, 2, 1
+
+
+@pytest.mark.parametrize("call,prefill", [
+    ((Q6_K, 32, 2048, 2048), False), ((Q6_K, 48, 2048, 2048), True), ((Q4_K, 64, 896, 1024), False),
+    ((Q4_K, 128, 896, 1024), True), ((Q6_K, 128, 512, 512), False), ((Q6_K, 256, 512, 512), True),
+    ((Q4_0, 24, 64, 8192), True), ((F16, 40, 64, 1024), False), ((F16, 48, 64, 1024), True),
+    ((Q8_0, 24, 2048, 2048), True), ((Q4_K, 127, 3072, 3072), True), ((Q6_K, 23, 3072, 3072), False)])
+def test_small_prompt_calls_take_the_faster_kernels(fake, call, prefill):
+    """Both sides of the line between the verify and the prefill kernels."""
+    got = any("k_pf" in line for line in fake("gemm", *call))
+    assert got == prefill
+
+
+def test_the_prefill_kernels_tests_reach_them(fake):
+    """Cases of the GPU tests that are there for the prefill kernels."""
+    import test_gpu_prefill as t
+
+    for qt, nt, n_out, n_in in t.K_CASES + [c for c in t.CASES if c[0] in (Q8_0, Q4_0)]:
+        assert any("k_pfI" in line for line in fake("gemm", qt, nt, n_out, n_in)), (qt, nt, n_out, n_in)
