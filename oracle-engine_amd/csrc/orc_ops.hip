@@ -1650,6 +1650,25 @@ static void attn_launch(bool timed, const LaunchEv& ev, K kernel, dim3 grid, dim
     else hipLaunchKernelGGL(kernel, grid, block, lds, st, args...);
 }
 
+// Whether a short context is one for k_attn_pf alone: its chain is a few
+// 64-position chunks (3.1 to 11.7 us each, growing with the query heads per kv
+// head R), where the split of K and V costs a launch. Only while its workgroups
+// fit the CUs in a round. Measured (us, k_attn_pf against the split; 64 tokens
+// at 0 unless said): 64-wide heads, R 1 9.6 and 12.6, 128 tokens 12.9 and 14.1,
+// at 60 16.1 and 15.5; R 2 10.8 and 12.3, 128 tokens 14.9 and 13.9; R 4 13.4
+// and 12.4, 8 tokens 11.1 and 11.7. 128-wide, R 1 12.4 and 17.4, 128 tokens at
+// 60 21.2 and 22.4, 256 at 0 27.3 and 24.9 (32 kv heads, 64 tokens at 300: 33.1
+// and 36.1); R 2 14.7 and 17.0, 128 tokens 20.5 and 19.5; R 3 16.9 and 17.0, 8
+// tokens 13.6 and 15.7.
+static bool attn_short(int n_tok, int n_heads, int n_kv, int head_dim, int p_end) {
+    const int R = n_heads / n_kv, few = n_tok <= 8;
+    if ((long)((n_tok + kPaTok - 1) / kPaTok) * n_kv > g_n_cu) return false;
+    int chunks = 0;  // at most
+    if (head_dim == 64) chunks = R == 1 ? 2 : R == 2 ? 1 : R <= 4 ? few : 0;
+    else chunks = R == 1 ? 3 + n_kv / 8 : R == 2 ? 1 + few : R == 3 ? few : 0;
+    return p_end <= chunks * kSB;
+}
+
 extern "C" int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_heads, int n_kv, int head_dim,
                                 int pos_off, const float* d_rope, float* d_kc, float* d_vc, int ctx, float* d_out,
                                 int ldo, orc_stream_t s) {
@@ -1670,7 +1689,9 @@ extern "C" int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_
     bytes += 4.0 * n_tok * ((double)(n_heads + 2 * n_kv) * head_dim + (double)n_heads * head_dim);
     LaunchEv ev;
     uint8_t* work = nullptr;
-    int rc = fa_bytes(head_dim, n_kv, pos_off + n_tok) <= kPfWorkBytes ? pf_ws_begin(st, &work) : kPfBusy;
+    const int p_end = pos_off + n_tok;
+    const bool split = !attn_short(n_tok, n_heads, n_kv, head_dim, p_end) && fa_bytes(head_dim, n_kv, p_end) <= kPfWorkBytes;
+    int rc = split ? pf_ws_begin(st, &work) : kPfBusy;
     if (rc && rc != kPfBusy) return rc;
     const bool tm = prof_arm(st, kProfAttnPf, n_tok, bytes, &ev.a, &ev.b);
     if (!rc) {

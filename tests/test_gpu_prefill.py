@@ -251,10 +251,12 @@ def test_token_chunks(dev, oracle):
 
 
 @pytest.mark.parametrize("H,KVH,hd,sp,nt", [(8, 1, 64, 0, 1), (7, 7, 128, 31, 33), (24, 8, 128, 4000, 30),
-                                            (28, 4, 128, 95, 129), (16, 2, 64, 640, 600)])
+                                            (28, 4, 128, 95, 129), (16, 2, 64, 640, 600), (7, 7, 128, 287, 33),
+                                            (3, 3, 64, 96, 33), (2, 2, 64, 60, 68), (8, 4, 128, 10, 54), (6, 2, 128, 56, 8)])
 def test_prefill_attention(dev, H, KVH, hd, sp, nt):
-    """The prefill attention over split K and V (csrc/orc_attn_pf.hip) against
-    float64: block edges of 32 positions, padded row tiles, key ranges merged
+    """The prefill attention (over split K and V, csrc/orc_attn_pf.hip, and
+    k_attn_pf for the short contexts of few query heads) against float64: block
+    edges of 32 positions, padded row tiles, key ranges merged
     over workgroups (few rows over a long cache), values whose scale differs by
     2^20 between key blocks and dimensions. Scores are fp32-like (2^-22 per
     product, |score| up to ~30): 4e-6 of the row's largest output. A repeat

@@ -66,3 +66,14 @@ def test_the_prefill_kernels_tests_reach_them(fake):
 
     for qt, nt, n_out, n_in in t.K_CASES + [c for c in t.CASES if c[0] in (Q8_0, Q4_0)]:
         assert any("k_pfI" in line for line in fake("gemm", qt, nt, n_out, n_in)), (qt, nt, n_out, n_in)
+
+
+@pytest.mark.parametrize("call,split", [
+    ((8, 8, 64, 64, 0), False), ((8, 8, 64, 128, 0), False), ((8, 8, 64, 129, 0), True), ((16, 8, 64, 64, 0), False),
+    ((16, 8, 64, 65, 0), True), ((32, 8, 64, 8, 56), False), ((32, 8, 64, 9, 50), True), ((14, 2, 64, 4, 0), True),
+    ((8, 8, 128, 64, 192), False), ((8, 8, 128, 64, 193), True), ((32, 32, 128, 64, 384), False),
+    ((32, 32, 128, 129, 0), True), ((16, 8, 128, 8, 100), False), ((16, 8, 128, 16, 100), True),
+    ((24, 8, 128, 8, 50), False), ((24, 8, 128, 24, 0), True), ((28, 4, 128, 1, 0), True)])
+def test_short_contexts_take_the_faster_attention(fake, call, split):
+    """heads, kv heads, head_dim, tokens, position: both sides of the line."""
+    assert any("k_kv_split" in line for line in fake("attn", *call)) == split
