@@ -918,12 +918,13 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
 //    rows are cut at 16 superblocks at any size: the rounding of one long
 //    chain would exceed the fp32 kernel's (8192 values: 1.35e-7 of the
 //    result in one range, 1.1e-7 in two, 1.33e-7 there).
+constexpr int kDenseSupers = 16;
+static bool pf_dense(int type) { return type == ORC_F16 || type == ORC_BF16; }
 struct PfPlan {
     int shape, nz;  // shape 0: 128 x 128, 1: 128 x 64, 2: 128 x 32
 };
 static PfPlan pf_plan(int type, const QmvParams& p, int supers) {
     const int rows = p.epi == ORC_EPI_SWIGLU ? 2 * p.rows[0] : p.n_rows;
-    const bool dense = type == ORC_F16 || type == ORC_BF16;
     auto wgs = [&](int bt) { return (long)((rows + 127) / 128) * ((p.n_tok + bt - 1) / bt); };
     PfPlan r{1, 1};
     const int most = std::min(16, std::max(1, (supers + 1) / (p.n_tok <= 128 ? 2 : 3)));
@@ -934,7 +935,7 @@ static PfPlan pf_plan(int type, const QmvParams& p, int supers) {
     else
         r.nz = (int)std::min<long>(most, 3 * g_n_cu / wgs(r.shape == 0 ? 128 : 64));
     r.nz = std::max(r.nz, 1);
-    if (dense) r.nz = std::max(r.nz, (supers + 15) / 16);
+    if (pf_dense(type)) r.nz = std::max(r.nz, (supers + kDenseSupers - 1) / kDenseSupers);
     return r;
 }
 
@@ -987,14 +988,25 @@ static int pf_split(const PfType& t, const PfSplit& sp, int ng, hipStream_t s, h
     return ORC_OK;
 }
 
+// Tokens of a chunk: as many as fit the workspace, with the partial sums of the
+// ranges that a long F16 or BF16 row needs (a chunk of fewer tokens otherwise,
+// down to 64; 0: not even those). Other partial sums take what is left.
+static int pf_chunk(int type, const PfType& t, const QmvParams& p) {
+    PfWork w;
+    const int supers = (p.n_in + kSuper - 1) / kSuper, nz = pf_dense(type) ? (supers + kDenseSupers - 1) / kDenseSupers : 1;
+    const size_t tok = nz > 1 ? (size_t)nz * p.n_rows * sizeof(float) : 0;
+    const size_t per = pf_layout(t, p.n_in, 4, nullptr, w) + 128 * tok;
+    if (per <= kPfWorkBytes) return (int)std::min<size_t>(kPfWorkBytes / per, 1 << 20) * 128;
+    return pf_layout(t, p.n_in, 2, nullptr, w) + 64 * tok <= kPfWorkBytes ? 64 : 0;
+}
+
 bool pf_takes(int type, const QmvParams& p) {
     if (p.n_tok < kPfSplitMin || p.n_in % 32) return false;
     PfType t;
     if (type == kMixK) t = {2, true, true};
     else if (!pf_type(type, t)) return false;
     if (p.epi == ORC_EPI_SWIGLU && p.n_seg != 2) return false;
-    PfWork w;
-    return pf_layout(t, p.n_in, 4, nullptr, w) <= kPfWorkBytes;
+    return pf_chunk(type, t, p) > 0;
 }
 
 int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& ev, uint8_t* buf) {
@@ -1002,8 +1014,7 @@ int pf_launch(int type, const QmvParams& p0, hipStream_t s, const LaunchEvents& 
     if (type == kMixK) t = {2, true, true};  // Q4_K and Q6_K segments share one split
     else if (!pf_type(type, t)) return set_error(ORC_E_INVALID, "gemm: not a prefill launch");
     PfWork w;
-    const size_t per4 = pf_layout(t, p0.n_in, 4, nullptr, w);  // 128 tokens
-    const int chunk = (int)std::min<size_t>(kPfWorkBytes / per4, 1 << 20) * 128;
+    const int chunk = pf_chunk(type, t, p0);
     int rc = ORC_OK;
     for (int t0 = 0; t0 < p0.n_tok && !rc; t0 += chunk) {
         QmvParams p = p0;

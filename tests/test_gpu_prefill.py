@@ -489,3 +489,22 @@ def test_prefill_attention_infinities_reach_no_earlier_token(dev, H, KVH, hd, nt
     V2[:, 40, 5] = np.inf
     got, _, _ = _attn_case(dev, H, KVH, hd, sp, nt, S, K, V2, qkv.reshape(nt, -1))
     assert np.isposinf(got[:, :, 5]).all() and np.isfinite(np.delete(got, 5, 2)).all()
+
+
+def test_tall_dense_matrix_in_chunks(dev, oracle):
+    """A tall F16 matrix of long rows: the sums of its two ranges leave room
+    for 64 tokens at a time. 262144 rows that repeat 64."""
+    print("[gpu] pf tall F16 262144 x 8192, 130 tokens", flush=True)
+    rng = np.random.default_rng(14)
+    n_in, base, n_out, nt = 8192, 64, 262144, 130
+    w, ty, W = _weights(dev, oracle, ol.F16, base, n_in, rng)
+    big = dev.alloc(n_out * n_in * 2)
+    done = base * n_in * 2
+    dev.check(dev.L.orc_memcpy_d2d(big.ptr, w.ptr, done, None))
+    while done < n_out * n_in * 2:
+        dev.check(dev.L.orc_memcpy_d2d(big.ptr + done, big.ptr, done, None))
+        done *= 2
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    got = _gemm(dev, ty, big, X, n_out).reshape(nt, -1, base)
+    _check(got[:, 0], X, W)
+    assert (got == got[:, :1]).all()

@@ -77,3 +77,15 @@ def test_the_prefill_kernels_tests_reach_them(fake):
 def test_short_contexts_take_the_faster_attention(fake, call, split):
     """heads, kv heads, head_dim, tokens, position: both sides of the line."""
     assert any("k_kv_split" in line for line in fake("attn", *call)) == split
+
+
+@pytest.mark.parametrize("call,ranges", [((F16, 300, 128256, 8192), 2), ((F16, 3000, 128256, 8192), 2),
+                                         ((30, 200, 128256, 12288), 3), ((F16, 300, 400000, 8192), 2),
+                                         ((F16, 300, 700000, 8192), 0)])
+def test_tall_dense_matrices_keep_their_ranges(fake, call, ranges):
+    """An F16 or BF16 row is summed in ranges of at most 4096 values however
+    much of the workspace their sums take: in chunks of fewer tokens, or (64
+    tokens do not fit) by the kernels that need no workspace."""
+    got = [int(line.split()[2].split("x")[2]) for line in fake("gemm", *call) if "4k_pfI" in line]
+    assert len(got) > 0 if ranges else not got
+    assert all(z >= ranges for z in got), got
