@@ -1000,12 +1000,16 @@ static int pf_chunk(int type, const PfType& t, const QmvParams& p) {
     return pf_layout(t, p.n_in, 2, nullptr, w) + 64 * tok <= kPfWorkBytes ? 64 : 0;
 }
 
+constexpr int kPfMaxRows = 65535 * 128;
+
 bool pf_takes(int type, const QmvParams& p) {
     if (p.n_tok < kPfSplitMin || p.n_in % 32) return false;
     PfType t;
     if (type == kMixK) t = {2, true, true};
     else if (!pf_type(type, t)) return false;
     if (p.epi == ORC_EPI_SWIGLU && p.n_seg != 2) return false;
+    // blocks of 128 rows (64 SwiGLU pairs) are the second grid dimension
+    if (p.n_rows > kPfMaxRows) return false;
     return pf_chunk(type, t, p) > 0;
 }
 

@@ -89,3 +89,9 @@ def test_tall_dense_matrices_keep_their_ranges(fake, call, ranges):
     got = [int(line.split()[2].split("x")[2]) for line in fake("gemm", *call) if "4k_pfI" in line]
     assert len(got) > 0 if ranges else not got
     assert all(z >= ranges for z in got), got
+
+
+@pytest.mark.parametrize("call", [(Q8_0, 24, 65535 * 128, 32), (Q8_0, 24, 65535 * 128 + 1, 32), (F16, 300, 9000000, 64),
+                                  (Q4_K, 40, 8400000, 256)])
+def test_any_number_of_rows_is_taken(fake, call):
+    fake("gemm", *call)
