@@ -58,7 +58,7 @@ typedef void* orc_event_t;  /* a hipEvent_t */
 
 /* ── runtime ─────────────────────────────────────────────────────────────── */
 /* Select `device`, create the default stream and allocate the workspace of
- * the prefill GEMM and attention (256 MB of device memory, shared by every
+ * the prefill GEMM and attention (264 MB of device memory, shared by every
  * call on the device and freed by orc_shutdown; without that much free memory
  * those calls run slower kernels that need none). Replaces nothing in the
  * reference (CPU-only); called once by the host before any other entry point. */

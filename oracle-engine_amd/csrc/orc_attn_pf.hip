@@ -608,6 +608,9 @@ template <int HD> static int fa_run(const FaArgs& a, uint8_t* buf, size_t cap, h
     return ORC_OK;
 }
 
+static_assert(8 * (32768 / kKB) * (fa_block_bytes<128>() + sizeof(int)) + 256 * 32 * (128 + 4) * sizeof(float) <= kPfWorkBytes,
+              "32 K positions of eight 128-wide kv heads and their key ranges");
+
 size_t fa_bytes(int hd, int n_kv, int p_end) {
     const size_t n = (size_t)n_kv * ((p_end + kKB - 1) / kKB);
     return (n * (hd * 256 + sizeof(int)) + 255) / 256 * 256;

@@ -73,12 +73,13 @@ int pf_init();
 void pf_release();
 // The workspace of the prefill kernels (one per device): 1024 tokens of 18944
 // split values (83 MB) with room for partial sums, or the split K and V of
-// 32 K positions of eight 128-wide kv heads. pf_ws_begin locks it and orders
+// 32 K positions of eight 128-wide kv heads (256 MB and a word per block) with
+// the partial results of 32 rows in each of 256 workgroups (4.3 MB). pf_ws_begin locks it and orders
 // the stream behind its last use; kPfBusy where the caller takes a path
 // without it: the stream is being captured, there is no workspace, or its last
 // use was on a library stream whose capture was begun through HIP itself
 // instead of orc_graph_begin. pf_ws_end ends the use and unlocks.
-constexpr size_t kPfWorkBytes = (size_t)256 << 20;
+constexpr size_t kPfWorkBytes = (size_t)264 << 20;
 constexpr int kPfBusy = 1;
 int pf_ws_begin(hipStream_t s, uint8_t** buf);
 int pf_ws_end(hipStream_t s);

@@ -198,7 +198,7 @@ static void capture_order() {
     CHECK(!orc_graph_end(a, &g) && !orc_stream_destroy(a) && !orc_stream_destroy(b));
 }
 
-// A device that has no 256 MB left: orc_init and every call work, on the
+// A device without the memory for the workspace: orc_init and every call work, on the
 // kernels that need no workspace.
 static void no_memory() {
     malloc_limit = 100 << 20;

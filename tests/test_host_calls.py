@@ -95,3 +95,12 @@ def test_tall_dense_matrices_keep_their_ranges(fake, call, ranges):
                                   (Q4_K, 40, 8400000, 256)])
 def test_any_number_of_rows_is_taken(fake, call):
     fake("gemm", *call)
+
+
+def test_the_workspace_holds_32_k_positions(fake):
+    """The last pass of a 32768-position prompt of eight 128-wide kv heads, and
+    its key ranges over few rows."""
+    for call in ((32, 8, 128, 1024, 31744), (32, 8, 128, 40, 32728), (64, 8, 128, 1, 32767)):
+        got = fake("attn", *call)
+        assert any("k_kv_split" in line for line in got), call
+    assert any("k_attn_fa_sum" in line for line in got)
