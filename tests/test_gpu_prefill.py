@@ -508,3 +508,98 @@ def test_tall_dense_matrix_in_chunks(dev, oracle):
     got = _gemm(dev, ty, big, X, n_out).reshape(nt, -1, base)
     _check(got[:, 0], X, W)
     assert (got == got[:, :1]).all()
+
+
+def _captured(dev, call, outs, runs=3):
+    """call(stream) captured on a stream of its own and replayed `runs` times,
+    with eager work between; the outputs of every replay are the same bits."""
+    s, graph = C.c_void_p(), C.c_void_p()
+    dev.check(dev.L.orc_stream_create(C.byref(s)))
+    dev.check(dev.L.orc_graph_begin(s))
+    call(s)
+    dev.check(dev.L.orc_graph_end(s, C.byref(graph)))
+    got = []
+    for _ in range(runs):
+        for o in outs:
+            dev.check(dev.L.orc_fill(o.ptr, 0xFF, o.nbytes, s))
+        dev.check(dev.L.orc_graph_launch(graph, s))
+        dev.sync()
+        got.append([o.read(np.float32) for o in outs])
+        call(None)  # the same call eagerly, over the workspace
+        dev.sync()
+    for g in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
+    dev.check(dev.L.orc_graph_destroy(graph))
+    dev.check(dev.L.orc_stream_destroy(s))
+    return got[0]
+
+
+@pytest.mark.parametrize("qt,nt,n_out,n_in", [(ol.Q4_K, 300, 300, 3072), (ol.Q6_K, 263, 200, 18944), (ol.Q6_K, 256, 130, 2048),
+                                              (ol.Q8_0, 263, 200, 896), (ol.Q8_0, 256, 70, 4864),
+                                              (ol.Q8_0_X8, 256, 257, 3072), (ol.Q4_0, 256, 40, 1120), (ol.F16, 260, 40, 512)])
+def test_captured_prefill_gemm(dev, oracle, qt, nt, n_out, n_in):
+    """Captured calls of 256 tokens and more: k_mmq_pf for the K-quants and
+    Q8_0 (64 tokens per workgroup), the vector kernels' token blocks else."""
+    print(f"[gpu] captured gemm type={qt} nt={nt} {n_out}x{n_in}", flush=True)
+    rng = np.random.default_rng(nt + n_in)
+    w, ty, W = _weights(dev, oracle, qt, n_out, n_in, rng)
+    X = rng.normal(0, 1, (nt, n_in)).astype(np.float32)
+    dx, dy = dev.upload(X), dev.alloc(nt * n_out * 4)
+    got, = _captured(dev, lambda s: dev.check(dev.L.orc_gemm(ty, w.ptr, nt, n_out, n_in, dx.ptr, n_in, dy.ptr, n_out, s)), [dy])
+    _check(got.reshape(nt, n_out), X, W)
+
+
+@pytest.mark.parametrize("qt", [ol.Q4_K, ol.Q6_K, ol.Q8_0])
+def test_captured_prefill_epilogues(dev, oracle, qt):
+    """k_mmq_pf's norm, bias, SwiGLU (Q8_0: two passes over the output) and
+    residual sums against float64; no pass reads what a replay before it left."""
+    import orc
+
+    rng = np.random.default_rng(20)
+    nt, n_in, rows = 300, 1024, (144, 80)
+    ws = [_weights(dev, oracle, qt, r, n_in, rng) for r in rows]
+    X = rng.normal(0, 2, (nt, n_in)).astype(np.float32)
+    g, bias = rng.uniform(0.5, 1.5, n_in).astype(np.float32), rng.normal(0, 1, rows[1]).astype(np.float32)
+    dx, dg, db, dy, dh = dev.upload(X), dev.upload(g), dev.upload(bias), dev.alloc(nt * sum(rows) * 4), dev.alloc(nt * 80 * 4)
+    print(f"[gpu] captured epilogues type={qt}", flush=True)
+
+    def call(s):
+        segs = (orc.Seg * 2)(orc.Seg(ws[0][0].ptr, rows[0], dy.ptr, None), orc.Seg(ws[1][0].ptr, rows[1], dy.ptr + 4 * rows[0], db.ptr))
+        dev.check(dev.L.orc_gemm_fused(qt, segs, 2, nt, n_in, dx.ptr, n_in, sum(rows), dg.ptr, C.c_float(1e-5), orc.EPI_STORE, s))
+        segs = (orc.Seg * 2)(orc.Seg(ws[0][0].ptr, 80, dh.ptr, None), orc.Seg(ws[1][0].ptr, 80, dh.ptr, None))
+        dev.check(dev.L.orc_gemm_fused(qt, segs, 2, nt, n_in, dx.ptr, n_in, 80, dg.ptr, C.c_float(1e-5), orc.EPI_SWIGLU, s))
+        segs = (orc.Seg * 1)(orc.Seg(ws[1][0].ptr, 80, dh.ptr, None))
+        dev.check(dev.L.orc_gemm_fused(qt, segs, 1, nt, n_in, dx.ptr, n_in, 80, None, C.c_float(0), orc.EPI_ACCUM, s))
+
+    y, h = _captured(dev, call, [dy, dh])
+    Xd = X.astype(np.float64)
+    Xn = Xd / np.sqrt((Xd ** 2).mean(1, keepdims=True) + 1e-5) * g
+    dot, scale = [Xn @ w[2].T for w in ws], [np.abs(Xn) @ np.abs(w[2]).T for w in ws]
+    want = np.concatenate([dot[0], dot[1] + bias], 1)
+    assert np.all(np.abs(y.reshape(nt, -1) - want) <= 2e-6 * np.concatenate(scale, 1) + 3e-7 * np.abs(want))
+    gt, up = dot[0][:, :80], dot[1]
+    act = gt / (1 + np.exp(-gt)) * up
+    res = Xd @ ws[1][2].T
+    tol = 3e-6 * (scale[0][:, :80] * np.abs(up) + scale[1] * np.abs(gt)) + 2e-6 * (np.abs(Xd) @ np.abs(ws[1][2]).T) + 1e-6 * np.abs(act)
+    assert np.all(np.abs(h.reshape(nt, -1) - (act + res)) <= tol)  # |silu'| <= 1.1
+
+
+@pytest.mark.parametrize("H,KVH,hd,sp,nt", [(8, 2, 128, 500, 70), (14, 2, 64, 700, 33)])
+def test_captured_attention_of_long_contexts(dev, H, KVH, hd, sp, nt):
+    """k_attn_pf, which an eager call of these sizes does not take, against
+    the eager call: both within 4e-6 of float64 (the largest output)."""
+    print(f"[gpu] captured attention H={H} KVH={KVH} hd={hd} sp={sp} nt={nt}", flush=True)
+    rng = np.random.default_rng(sp)
+    ctx, ld = sp + nt, (H + 2 * KVH) * hd
+    qkv = rng.normal(0, 1, (nt, ld)).astype(np.float32)
+    K, V = (rng.normal(0, 1, (KVH, ctx, hd)).astype(np.float32) for _ in range(2))
+    th = np.arange(ctx)[:, None] / 1e4 ** (np.arange(hd // 2) * 2.0 / hd)
+    dt = dev.upload(np.stack([np.cos(th), np.sin(th)], -1).astype(np.float32))
+    dq, dK, dV, do = dev.upload(qkv), dev.upload(K), dev.upload(V), dev.alloc(nt * H * hd * 4)
+
+    def call(s):
+        dev.check(dev.L.orc_attn_prefill(dq.ptr, ld, nt, H, KVH, hd, sp, dt.ptr, dK.ptr, dV.ptr, ctx, do.ptr, H * hd, s))
+
+    got, = _captured(dev, call, [do])
+    want = do.read(np.float32)  # the last eager call's
+    assert np.allclose(got, want, rtol=0, atol=8e-6 * np.abs(want).max())
