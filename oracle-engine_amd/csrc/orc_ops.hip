@@ -1683,16 +1683,17 @@ extern "C" int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_
     const int R = n_heads / n_kv;
     hipStream_t st = resolve_stream(s);
     const dim3 grid((n_tok + kPaTok - 1) / kPaTok, n_kv);
-    double bytes = 0;  // K / V rows of every query block's positions, once per block; QKV rows in, rows out
-    for (int t0 = 0; t0 < n_tok; t0 += kPaTok)
-        bytes += 8.0 * n_kv * head_dim * (pos_off + std::min(n_tok, t0 + kPaTok));
-    bytes += 4.0 * n_tok * ((double)(n_heads + 2 * n_kv) * head_dim + (double)n_heads * head_dim);
     LaunchEv ev;
     uint8_t* work = nullptr;
     const int p_end = pos_off + n_tok;
     const bool split = !attn_short(n_tok, n_heads, n_kv, head_dim, p_end) && fa_bytes(head_dim, n_kv, p_end) <= kPfWorkBytes;
     int rc = split ? pf_ws_begin(st, &work) : kPfBusy;
     if (rc && rc != kPfBusy) return rc;
+    // K / V rows once (k_attn_pf: once per query block), QKV rows in, rows out
+    double bytes = 4.0 * n_tok * ((double)(n_heads + 2 * n_kv) * head_dim + (double)n_heads * head_dim);
+    if (!rc) bytes += 8.0 * n_kv * head_dim * p_end;
+    else
+        for (int t0 = 0; t0 < n_tok; t0 += kPaTok) bytes += 8.0 * n_kv * head_dim * (pos_off + std::min(n_tok, t0 + kPaTok));
     const bool tm = prof_arm(st, kProfAttnPf, n_tok, bytes, &ev.a, &ev.b);
     if (!rc) {
         const FaArgs a{d_qkv, ldqkv, n_tok, n_heads, n_kv, pos_off, (const float2*)d_rope, d_kc, d_vc, ctx, d_out, ldo, st};

@@ -121,6 +121,9 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { return *e = nullptr, hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = (hipEvent_t) new Event, hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete (Event*)e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     LOCK;
@@ -221,6 +224,29 @@ static void route(int argc, char** argv) {
         CHECK(!orc_attn_prefill(X, (v[0] + 2 * v[1]) * v[2], v[3], v[0], v[1], v[2], v[4], X, X, X, v[4] + v[3], X, v[0] * v[2], nullptr));
 }
 
+// The bytes noted for timed attention calls: K and V once, QKV rows in, rows
+// out, over the workspace; k_attn_pf reads K and V once per 16-token block.
+static void prof_bytes() {
+    const int H = 28, KV = 4, hd = 128, n = 1023, pos = 7168, ld = (H + 2 * KV) * hd;
+    CHECK(!orc_init(0));
+    auto bytes = [&] {
+        int64_t calls = 0;
+        double ms = 0, by = 0;
+        orc_prof_enable(1);
+        CHECK(!orc_attn_prefill(X, ld, n, H, KV, hd, pos, X, X, X, pos + n, X, H * hd, nullptr));
+        CHECK(!orc_prof_accumulate() && !orc_prof_read(ORC_PROF_ATTN_PF, n, &calls, &ms, &by) && calls == 1);
+        orc_prof_enable(0);
+        return by;
+    };
+    const double rows = 4.0 * n * (ld + H * hd), kv = 8.0 * KV * hd;
+    CHECK(bytes() == kv * (pos + n) + rows);
+    double all = 0;
+    for (int t = 0; t < n; t += 16) all += kv * (pos + (t + 16 < n ? t + 16 : n));
+    CHECK(!orc_shutdown());
+    malloc_limit = 100 << 20;
+    CHECK(!orc_init(0) && bytes() == all + rows);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc > 1);
     const std::string w = argv[1];
@@ -228,6 +254,7 @@ int main(int argc, char** argv) {
     else if (w == "race_hip") capture_race(false);
     else if (w == "order") capture_order();
     else if (w == "no_memory") no_memory();
+    else if (w == "prof_bytes") prof_bytes();
     else if (w == "gemm" || w == "attn") route(argc, argv);
     else CHECK(!"a scenario");
     for (const std::string& l : launches) std::puts(l.c_str());

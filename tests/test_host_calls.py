@@ -104,3 +104,7 @@ def test_the_workspace_holds_32_k_positions(fake):
         got = fake("attn", *call)
         assert any("k_kv_split" in line for line in got), call
     assert any("k_attn_fa_sum" in line for line in got)
+
+
+def test_bytes_of_timed_attention_calls(fake):
+    fake("prof_bytes")
