@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <unordered_set>
 
 namespace orc {
@@ -149,9 +150,10 @@ extern "C" int orc_stream_create(orc_stream_t* s) {
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
     hipStream_t st;
     ORC_HIP_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    {
+    try {
         std::lock_guard<std::mutex> lk(g_streams_mu);
         g_streams.insert(st);
+    } catch (const std::bad_alloc&) {  // then it is treated as a stream of the caller's own
     }
     *s = (orc_stream_t)st;
     return ORC_OK;

@@ -34,6 +34,7 @@
 
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <unordered_set>
 
 namespace orc {
@@ -1799,12 +1800,21 @@ static std::unordered_set<const void*> g_all_tokens;
 // once. Only a hint: either route samples any state as its parameters say.
 static std::unordered_set<const void*> g_one_wg;
 
-static void note_params(const void* d_state, float temperature, int top_k) {
+// False: no host memory to note a state whose rows have a limit.
+static bool note_params(const void* d_state, float temperature, int top_k) {
     std::lock_guard<std::mutex> lk(g_all_mu);
-    if (top_k == 0 && temperature > 0.f) g_all_tokens.insert(d_state);  // T <= 0 sorts nothing (argmax)
-    else g_all_tokens.erase(d_state);
-    if (temperature > 0.f && top_k >= 1 && top_k <= kTxK) g_one_wg.erase(d_state);
-    else g_one_wg.insert(d_state);
+    try {
+        if (top_k == 0 && temperature > 0.f) g_all_tokens.insert(d_state);  // T <= 0 sorts nothing (argmax)
+        else g_all_tokens.erase(d_state);
+    } catch (const std::bad_alloc&) {
+        return false;
+    }
+    try {
+        if (temperature > 0.f && top_k >= 1 && top_k <= kTxK) g_one_wg.erase(d_state);
+        else g_one_wg.insert(d_state);
+    } catch (const std::bad_alloc&) {  // without the hint orc_sample takes the split route, which does as the parameters say
+    }
+    return true;
 }
 
 static int check_vocab(const void* d_state, int n_vocab, const char* who) {
@@ -1841,7 +1851,7 @@ extern "C" int orc_sampler_init(void* d_state, float temperature, float top_p, i
     if (!d_state || repeat_last < 0 || repeat_last >= kSampHist || n_hist < 0 || (n_hist && !d_hist) ||
         top_k < 0 || top_k > kCandMax)
         return set_error(ORC_E_INVALID, "sampler_init: bad args (0 <= top_k <= 16384, 0 <= repeat_last < 4096)");
-    note_params(d_state, temperature, top_k);
+    if (!note_params(d_state, temperature, top_k)) return ORC_E_HIP;
     hipLaunchKernelGGL(k_sampler_init, dim3(1), dim3(64), 0, resolve_stream(s), (DevSampler*)d_state,
                        (uint32_t)seed, temperature, top_p, repeat_penalty, top_k, repeat_last, d_hist, n_hist);
     ORC_LAUNCH_CHECK();
@@ -1853,7 +1863,7 @@ extern "C" int orc_sampler_set_params(void* d_state, float temperature, float to
     if (!initialized()) return set_error(ORC_E_NOINIT, "orc_init not called");
     if (!d_state || repeat_last < 0 || repeat_last >= kSampHist || top_k < 0 || top_k > kCandMax)
         return set_error(ORC_E_INVALID, "sampler_set_params: bad args (0 <= top_k <= 16384, 0 <= repeat_last < 4096)");
-    note_params(d_state, temperature, top_k);
+    if (!note_params(d_state, temperature, top_k)) return ORC_E_HIP;
     hipLaunchKernelGGL(k_sampler_set, dim3(1), dim3(64), 0, resolve_stream(s), (DevSampler*)d_state, 1, temperature,
                        top_p, repeat_penalty, top_k, repeat_last);
     ORC_LAUNCH_CHECK();

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -45,11 +46,30 @@ static thread_local dim3 cfg_g, cfg_b;
 static thread_local size_t cfg_l;
 static thread_local hipStream_t cfg_s;
 
+static std::vector<hipStream_t> held;  // made beforehand
+static void hold_streams(hipStream_t* s, int n) { held.assign(s, s + n); }
+
 static Stream* S(hipStream_t s) { return (Stream*)s; }
 #define LOCK std::lock_guard<std::recursive_mutex> lk(mu)
 
+// operator new of the library too: fails while asked to
+static std::atomic<bool> no_new{false};
+void* operator new(size_t n) {
+    if (no_new) throw std::bad_alloc();
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+struct MayNew {  // this program's own notes
+    bool was = no_new.exchange(false);
+    ~MayNew() { no_new = was; }
+};
+
 static hipError_t launch(const void* f, dim3 g, hipStream_t s) {
     LOCK;
+    MayNew may;
     Dl_info info{};
     const char* n = dladdr(f, &info) && info.dli_sname ? info.dli_sname : "?";
     char line[600];
@@ -97,6 +117,7 @@ hipError_t hipMalloc(void** p, size_t n) {
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     static int n;
+    if (!held.empty()) return *s = held.back(), held.pop_back(), hipSuccess;
     return *s = (hipStream_t) new Stream{std::string(1, "0ABCDEFG"[n++ % 8])}, hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) { return delete S(s), hipSuccess; }
@@ -247,6 +268,23 @@ static void prof_bytes() {
     CHECK(!orc_init(0) && bytes() == all + rows);
 }
 
+// No exception leaves a C entry point where the host's memory runs out: the
+// library's own notes of streams and sampler states are left out.
+static void no_host_memory() {
+    CHECK(!orc_init(0));
+    hipStream_t pre[3];
+    for (hipStream_t& s : pre) hipStreamCreateWithFlags(&s, 0);
+    hold_streams(pre, 3);
+    no_new = true;
+    orc_stream_t a = nullptr;
+    const int rc = orc_stream_create(&a), rs = orc_sampler_init(X, 0.f, 1.f, 0, 1.f, 0, 1, nullptr, 0, a);
+    no_new = false;
+    CHECK(!rc && a && !rs);
+    CHECK(!gemm(ORC_F16, 300, 2048, 2048, a) && !gemm(ORC_F16, 300, 2048, 2048, nullptr));  // an event after every use
+    CHECK(waits.size() == 1 && waits[0].e.on == S((hipStream_t)a));
+    CHECK(!orc_sample(X, X, 1000, (int32_t*)X, a) && !orc_stream_destroy(a));
+}
+
 int main(int argc, char** argv) {
     CHECK(argc > 1);
     const std::string w = argv[1];
@@ -255,6 +293,7 @@ int main(int argc, char** argv) {
     else if (w == "order") capture_order();
     else if (w == "no_memory") no_memory();
     else if (w == "prof_bytes") prof_bytes();
+    else if (w == "no_host_memory") no_host_memory();
     else if (w == "gemm" || w == "attn") route(argc, argv);
     else CHECK(!"a scenario");
     for (const std::string& l : launches) std::puts(l.c_str());

@@ -108,3 +108,7 @@ def test_the_workspace_holds_32_k_positions(fake):
 
 def test_bytes_of_timed_attention_calls(fake):
     fake("prof_bytes")
+
+
+def test_no_exception_leaves_a_c_entry_point(fake):
+    fake("no_host_memory")
