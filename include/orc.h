@@ -39,7 +39,7 @@ extern "C" {
 /* GGML type ids (core/gguf_parser.hpp:9-24) */
 #define ORC_F32 0
 #define ORC_F16 1
-#define ORC_BF16 30 /* dense weights: F32, F16 and BF16 rows run the vector GEMV */
+#define ORC_BF16 30 /* dense weights: F32, F16 and BF16 rows */
 #define ORC_Q4_0 2
 #define ORC_Q8_0 8
 #define ORC_Q4_K 12
@@ -119,8 +119,15 @@ int orc_embed(int type, const void* d_table, int n_in, int n_rows, const int32_t
  * the per-(token,row) reduction order does not depend on n_tok, so a verify
  * pass is bit-identical to n_tok separate GEMVs (Q4_K / Q6_K: to other calls
  * of two or more tokens). Calls of 24 tokens or more (prompt passes) of every
- * type but F32 run the matrix-core prefill kernels: within fp32 rounding of
- * the others, each token's row independent of the other tokens' values.
+ * type but F32 run the matrix-core prefill kernels, except over matrices so
+ * small that the others are faster: each token's row is independent of the
+ * other tokens' values, but its rounding (not its precision) depends on the
+ * call's token count and shape. There the activations are two fp16 halves
+ * with a power of two per token and 256 values (22 bits; a value more than
+ * 2^17 below the largest of its 256 keeps fewer; BF16 weights: 24 bits), and
+ * the error against exact products is no larger than the other kernels'.
+ * These calls share the library's workspace: calls on two streams run one
+ * after the other, a captured call runs kernels that need none.
  * Supported types: Q4_0, Q8_0, Q4_K, Q6_K, and the dense F32, F16 and BF16
  * (n_in a multiple of 32), which the reference runs through its dequantize +
  * ops::matmul fallback (core/model.cpp:370-381): fp32 sums over the exactly
@@ -164,11 +171,13 @@ int orc_gemm_fused_mixed(const int* types, const orc_seg* segs, int n_segs, int 
  * loops with std::chrono, bench_engine.cpp:225-244). While enabled, every
  * GEMM launch made outside stream capture carries a start and a stop HIP
  * event (hipExtLaunchKernelGGL: both take the timestamps of the kernel's own
- * dispatch on its stream) and its algorithmic HBM bytes (weight blocks + x +
- * y) are noted; so does every attention launch of orc_attn_fused_at with
+ * dispatch on its stream; a prefill call one pair around its two or three
+ * launches) and its algorithmic HBM bytes (weight blocks + x + y) are noted; so
+ * does every attention launch of orc_attn_fused_at with
  * host positions (families ORC_PROF_ATTN_WG / _MT / _SPLIT / _MERGE, and
- * orc_attn_prefill: ORC_PROF_ATTN_PF; bytes = the K
- * and V rows its tokens read, counted once, + QKV rows in + rows out; the
+ * orc_attn_prefill: ORC_PROF_ATTN_PF; bytes = the K and V rows its tokens
+ * read, counted once (in the one-launch prefill form once per 16-token block),
+ * + QKV rows in + rows out; the
  * merge is noted with 0 bytes). Once the work has run, orc_prof_accumulate
  * adds every launch's elapsed time to its record; orc_prof_read sums the
  * records of one kernel family (type = a GGML type id, 256 for mixed
@@ -282,13 +291,19 @@ int orc_attn_gqa_at(const float* d_q, int ldq, int n_tok, int n_heads, int n_kv,
  * calls take pos_floor = 0, pos_limit = ctx. */
 size_t orc_attn_fused_workspace(int n_heads, int n_kv, int head_dim);
 /* Prefill form of orc_attn_fused_at (host positions pos_off.., any n_tok, no
- * workspace): RoPE on q and k, K / V of every token stored in the cache,
- * causal attention of each token over positions 0..its own, written to
- * d_out (rows of ldo floats); the same layouts, limits (head_dim 64 / 128,
- * at most 8 query heads per kv head) and alignment. One workgroup per
- * (16-token block, kv head) walks the key chunks with an online softmax:
- * within fp32 rounding of orc_attn_fused_at's results, not equal to them
- * bit for bit (core/model.cpp:595-626 is the prefill counterpart). */
+ * workspace of the caller's): RoPE on q and k, K / V of every token stored in
+ * the cache, causal attention of each token over positions 0..its own,
+ * written to d_out (rows of ldo floats); the same layouts, limits (head_dim
+ * 64 / 128, at most 8 query heads per kv head) and alignment. Within fp32
+ * rounding of orc_attn_fused_at's results, not equal to them bit for bit
+ * (core/model.cpp:595-626 is the prefill counterpart). Two or three launches
+ * over the library's workspace, which holds the split K and V of the whole
+ * cache up to pos_off + n_tok (calls on two streams run one after the other);
+ * one launch without it inside a capture, for caches that do not fit (more
+ * than 32 K positions of eight 128-wide kv heads) and for short contexts of at
+ * most four query heads per kv head. K and V of any finite range keep fp32-like
+ * precision; an infinity or NaN in a V row reaches tokens from its position on
+ * (in the one-launch form also up to 15 before it). */
 int orc_attn_prefill(const float* d_qkv, int ldqkv, int n_tok, int n_heads, int n_kv, int head_dim, int pos_off,
                      const float* d_rope, float* d_kc, float* d_vc, int ctx, float* d_out, int ldo,
                      orc_stream_t stream);
@@ -343,7 +358,8 @@ int orc_sampler_init(void* d_state, float temperature, float top_p, int top_k, f
  * temperature, softmax, top-k, top-p, draw, record. Like the reference it
  * rewrites the row in place (it ends up holding the probabilities). T > 0 and
  * 1 <= top_k <= 128 on up to 196608 logits run split over many workgroups with
- * the state's scratch (calls on one state must not overlap). */
+ * the state's scratch (calls on one state must not overlap). A first draw, and
+ * one in 624, also refills the mt19937 state (70-85 us). */
 int orc_sample(void* d_state, float* d_logits, int n_vocab, int32_t* d_out, orc_stream_t stream);
 /* Sampler::record (sampler.cpp:99-105) of n device ids, in order. */
 int orc_sampler_record(void* d_state, const int32_t* d_tok, int n, orc_stream_t stream);

@@ -12,8 +12,11 @@
 //    lanes but one maximum per block.
 //  * k_attn_fa_sum merges key ranges where few rows leave CUs idle.
 // Products: hi x hi + hi x lo + lo x hi of exact fp16 halves, 3/16 of the time
-// of the fp32 MFMA chains this replaces (k_attn_pf, which stays for captured
-// calls and for caches larger than the workspace).
+// of the fp32 MFMA chains of k_attn_pf (which stays for captured calls, for
+// caches larger than the workspace and for short contexts, attn_short). Every
+// factor keeps ~22 bits against fp32's 24; the error against 64 bits is lower
+// all the same, since the sums are better (7B shape, 1023 tokens at 7168:
+// 3.9e-7 of the result against 1.65e-6).
 // Sums: the matrix cores round toward minus infinity, so every block's
 // products start from zero (the small ones apart for the scores, first for
 // P V), the blocks are added up in fp32 on the vector ALUs, and K and V are

@@ -817,8 +817,10 @@ __global__ __launch_bounds__(kSW) void k_attn_mt(const float* qkv, int ldqkv, in
 }
 
 // ── prefill attention: 16-token query blocks, no partials ───────────────────
-// orc_attn_prefill (prompt passes, host positions): one workgroup per (block
-// of kPaTok tokens, kv head g) carries the block's kPaTok x gqa rows
+// orc_attn_prefill (prompt passes, host positions) without the library's
+// workspace: inside a capture, for caches larger than it and for the short
+// contexts of attn_short (below); the others run k_kv_split and k_attn_fa
+// (orc_attn_pf.hip). One workgroup per (block of kPaTok tokens, kv head g) carries the block's kPaTok x gqa rows
 // (token-major) through every kSB-position key chunk up to the block's last
 // position with an online softmax (running max and sum per row in LDS), so
 // there are no partial rows and no merge launch, and a chunk's K / V rows are

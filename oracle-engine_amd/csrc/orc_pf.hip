@@ -18,20 +18,28 @@
 // (rows / 128 times over, more vector work than the products), and calls
 // below 256 tokens re-read and re-decoded the weights for each block of 5-16
 // tokens. Measured (MI355X, us before -> after): 7B gate+up Q6_K 37888 x 3584
-// at 1023 tokens 1790 -> 891 (2.8e14 products / s; at three MFMAs each 73% of
+// at 1023 tokens 1790 -> 891 (3.1e14 flop/s; at three MFMAs per product 74% of
 // what the card's bf16 library product reaches), at 127 tokens 741 -> 171;
 // 3B gate+up Q4_K 16384 x 3072 484 -> 304 and 178 -> 60; F16 16384 x 2048
 // 3168 -> 204 and 411 -> 45; 0.5B gate+up Q8_0 9728 x 896 236 -> 87. Error
 // against 64 bits: Q6_K 3584 values 1.1e-7 of the result's rms (1.2e-7 and
-// 1.6e-7 before), Q4_K 1.4e-7 (2.0e-7, 3.3e-7), Q8_0 1.0e-7 (3.9e-7).
+// 1.6e-7 before), Q4_K 1.4e-7 (2.0e-7, 3.3e-7), Q8_0 1.0e-7 (3.9e-7). Calls of
+// Q4_0, F16 and of 24 to 255 tokens of Q8_0 had fp32 activations before: over
+// 1B-shape blocks of 24 to 600 tokens Q4_0 2.2e-7 -> 1.0e-7, F16 1.4e-7 ->
+// 1.2e-7, Q8_0 3.9e-7 -> 1.1e-7 per product, the sums outweighing the two bits.
+// A value more than 2^17 below the largest of its token's 256 keeps fewer bits
+// than the others (14 at 2^24), as in the verify kernels of the K-quants.
 // What bounds k_pf: weight rows are read 32 bytes per lane pair (one cache
 // line per row and load: with all lanes on one row 7B gate+up took a third
 // less), the LDS reads of the fragments (1 KB per MFMA pair) and, at few
-// tokens, the latency of a stage.
+// tokens, the latency of a stage. GGUF Q8_0 and Q4_0 rows join their two block
+// scales as they are loaded, so a stage of theirs waits for the next one's
+// loads before its products (4.8 us a superblock of a lone chain against 2.7).
 //
 // The workspace between the two launches belongs to the library (one per
 // device, allocated by orc_init): calls take it in turn, ordered across
-// streams by an event. A call whose stream is being captured does not use it
+// streams by an event, so prefill calls on two streams do not overlap, and on a
+// stream the library did not create each is followed by an event (4.4 us). A call whose stream is being captured does not use it
 // (a graph could replay while another stream uses the workspace) and takes
 // the kernels that stage x themselves (orc_mmq.hip, orc_gemm.hip).
 #include "orc_gemm.hpp"
@@ -553,9 +561,11 @@ __global__ __launch_bounds__(64 * RW) __attribute__((amdgpu_waves_per_eu(2))) vo
     es_store(S0);
 
     // one stage: its fragments from the LDS against the row's codes, one
-    // (block, token tile) after another; a tile's fragments are read while
-    // the tile before multiplies. The scheduling barriers keep the compiler
-    // from starting more tiles at once than the registers hold.
+    // (block, token tile) after another; a tile's fragments are asked for ahead
+    // of the products of the tile before (the compiler moves the reads down to
+    // that tile's last product, which is all that covers them). The scheduling
+    // barriers keep it from starting more tiles at once than the registers
+    // hold.
     auto stage = [&](int st, int gb) {  // gb: first block of the stage in the granule
         const uint8_t* ab = sm + (st & 1) * kStageBytes + lane * 16;
         h8v av[2][2][PL], bh[2], bl[2];
@@ -909,8 +919,10 @@ static int pf_shape(const QmvParams& p, const PfWork& w, int nz, float* part, hi
 //    for BF16, whose three pieces per value leave one such workgroup per CU
 //    (332 against 262);
 //  * 128 x 64 otherwise (3072 x 3072 Q4_K, 1023 tokens: 84 against 107).
-//  * K is split while the tiles leave CUs idle: up to 768 workgroups, ranges
-//    of at least two superblocks (three above 128 tokens, where the partial
+//  * K is split while the tiles leave CUs idle: up to 768 workgroups (three
+//    per CU, which the 64-token kernels of Q4_K, Q8_0, Q4_0 and F16 allow; Q6_K
+//    and BF16 hold 177 and 172 registers, two per CU), ranges of at least two
+//    superblocks (three above 128 tokens, where the partial
 //    sums weigh more); with 32-token tiles up to 512 workgroups, and a short
 //    K in up to four ranges (896 x 896 at 256 tokens: 22.6, 18.6, 17.6 and
 //    16.1 in one to four). 3584 x 18944 at 127 tokens 364 in one range, 106 in

@@ -264,8 +264,8 @@ int Model::chunk_dev(const int32_t* d_ids, int n, const int32_t* d_pos, int sp, 
                            s));
         // RoPE + KV store (model.cpp:401-408), attention (model.cpp:410-435).
         // Prefill passes of kPrefillAttnMin tokens or more (host positions):
-        // one launch over the pass (query blocks, online softmax; the
-        // prefill attention of model.cpp:595-626). Otherwise launches of at
+        // the whole pass in one call (the prefill attention of
+        // model.cpp:595-626). Otherwise launches of at
         // most kMaxBatch tokens, in order: each stores its tokens' K / V rows
         // before the next attends to them.
         if (fused_attn_ && !d_pos && n >= kPrefillAttnMin) {

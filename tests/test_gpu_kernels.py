@@ -130,9 +130,9 @@ def test_gemm_batch_invariant(dev, oracle, qt, n_out, n_in):
                                               (ol.Q8_0_X8, 257, 3072, 256)])
 def test_gemm_prefill_vs_exact_and_blocks(dev, oracle, qt, n_out, n_in, nt):
     """Calls of 256 tokens or more on a K-quant or Q8_0 matrix run the
-    prefill kernel (64 tokens per workgroup, each weight slice decoded once
-    for all of them; Q8_0 from the GGUF blocks or the regrouped Q8_0_X8
-    layout, each block's scale applied to its own products): every (token,
+    prefill kernel over split activations (k_pf; Q8_0 from the GGUF blocks or
+    the regrouped Q8_0_X8 layout, each block's scale applied to its own
+    products; test_gpu_prefill.py has the captured form, k_mmq_pf): every (token,
     row) within 2e-6 of sum |w x| of the float64 product and within 4e-6 of
     the same tokens in 16-token calls (the verify path), with partial token
     and row blocks; a token's row does not depend on the call's other tokens
@@ -157,9 +157,9 @@ def test_gemm_prefill_vs_exact_and_blocks(dev, oracle, qt, n_out, n_in, nt):
 
 
 def test_gemm_prefill_epilogues(dev):
-    """The prefill kernel's RMSNorm prologue, bias, three output segments,
-    SwiGLU pairs and residual accumulation agree with the verify kernel's
-    (16-token calls of the same fused entry point)."""
+    """The prefill kernel's (k_pf) RMSNorm prologue, bias, three output
+    segments, SwiGLU pairs and residual accumulation agree with the verify
+    kernel's (16-token calls of the same fused entry point)."""
     print("[gpu] prefill gemm epilogues", flush=True)
     import orc
 
@@ -192,7 +192,7 @@ def test_gemm_prefill_epilogues(dev):
 
     a, b = both(qkv, ld)
     assert np.allclose(a, b, rtol=0, atol=2e-5 * np.abs(b).max())
-    for st in (ol.Q6_K, ol.Q4_K, ol.Q8_0):  # Q8_0: SwiGLU in two passes (gate rows, then up)
+    for st in (ol.Q6_K, ol.Q4_K, ol.Q8_0):
         wg, wu = (dev.upload(rand_blocks(st, ff * n_in, rng)) for _ in range(2))
 
         def swiglu(t0, n, dy):

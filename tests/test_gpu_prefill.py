@@ -1,15 +1,16 @@
 """The prefill GEMM over split activations (csrc/orc_pf.hip): calls of 24
 tokens and more on Q4_K, Q6_K, Q8_0 (GGUF and regrouped), Q4_0, F16 and BF16
-weights, against the float64 product of the oracle's dequantized rows.
+weights, against the float64 product of the oracle's dequantized rows; the
+kernels that captured calls of that size take; the prefill attention.
 
-Bound, per (token, row), relative to sum |w x|: 2^-22 for the activations'
-split, and 2^-24 per rounding of the sum: at most 12 in a 32-value block (two
-MFMA steps of up to three pieces, two roundings each), 8 blocks per 256 values,
-at most 16 superblocks in a range, 16 ranges and the norm's 1/rms: 1.2e-7 *
-(2 + 12 + 8 + 16 + 16) / ... stays under 2e-6 even if every rounding had the
-same sign, at magnitudes that grow with the partial sum (half of the worst
-case on average). The wider tests of the same entry points (256 tokens and
-more) use the same 2e-6.
+Bound of the GEMM, per (token, row), relative to sum |w x|: 2^-22 = 2.4e-7 for
+the activations' split; in a 32-value block at most 12 roundings of the matrix
+cores (two steps of up to three pieces, two roundings each) of 2^-23, which
+round toward minus infinity: 1.4e-6; 8 blocks per 256 values, 16 superblocks of
+a range and 16 ranges at 2^-24 each: 2.4e-6. That is 4.1e-6 if every rounding
+had its full size and one sign; but half of the blocks are stored negated and
+the roundings of the sums have either sign, so the tests hold 2e-6, as the wider
+tests of the same entry points (256 tokens and more) do.
 """
 import ctypes as C
 
