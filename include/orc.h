@@ -125,7 +125,9 @@ int orc_embed(int type, const void* d_table, int n_in, int n_rows, const int32_t
  * call's token count and shape. There the activations are two fp16 halves
  * with a power of two per token and 256 values (22 bits; a value more than
  * 2^17 below the largest of its 256 keeps fewer; BF16 weights: 24 bits), and
- * the error against exact products is no larger than the other kernels'.
+ * the error against exact products is no larger than the other kernels'. An
+ * infinite activation gives infinities or NaN in its own token's row, an
+ * infinite F16 or BF16 weight NaN.
  * These calls share the library's workspace: calls on two streams run one
  * after the other, a captured call runs kernels that need none.
  * Supported types: Q4_0, Q8_0, Q4_K, Q6_K, and the dense F32, F16 and BF16

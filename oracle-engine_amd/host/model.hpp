@@ -45,8 +45,8 @@ public:
     static constexpr int kPrefillBatch = 1024;  // tokens per device pass without logits (prefill)
     // Passes of this many tokens or more run orc_attn_prefill; below, three
     // or fewer 16-token launches of the verify path's attention are no slower
-    // (127 tokens of the 3B shape: 18 us against eight launches of 8 us; 24
-    // tokens: 19 against two).
+    // (127 tokens of the 3B shape: 19 us against eight launches of 8 us; 24
+    // tokens: 17 against two).
     static constexpr int kPrefillAttnMin = 48;
 
     Model() = default;
