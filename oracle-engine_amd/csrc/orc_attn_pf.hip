@@ -15,17 +15,17 @@
 // of the fp32 MFMA chains of k_attn_pf (which stays for captured calls, for
 // caches larger than the workspace and for short contexts, attn_short). Every
 // factor keeps ~22 bits against fp32's 24; the error against 64 bits is lower
-// all the same, since the sums are better (7B shape, 1023 tokens at 7168:
-// 3.9e-7 of the result against 1.65e-6).
+// all the same, since the sums are better (7B shape, 1023 tokens at 3000:
+// 2.8e-7 of the result against 1.14e-6; 3B, 127 at 0: 1.5e-7 against 2.7e-7).
 // Sums: the matrix cores round toward minus infinity, so every block's
 // products start from zero (the small ones apart for the scores, first for
 // P V), the blocks are added up in fp32 on the vector ALUs, and K and V are
 // stored negated in two of every four blocks.
 // Range: a block's probabilities are formed against its own row maximum
-// (rounded up to a power of two) and V against its own, so both halves of a
-// product hold their bits whatever the other blocks weigh; the running O and
-// sum keep their powers of two as integers, so adding a block up rounds
-// nothing but the sums themselves. Inside a block one power of two serves all
+// (rounded up to a whole power of two from the first block's) and V against its
+// own, so both halves of a product hold their bits whatever the other blocks
+// weigh; the running O and sum keep their powers of two as integers, so adding
+// a block up rounds nothing but the sums themselves. Inside a block one power of two serves all
 // 32 positions: a block where some K or V row's largest value is below 2^-16
 // of the block's (its halves would keep fewer than 22 bits), or that holds an
 // infinity or NaN (which must not reach rows that do not see the position: 0
@@ -305,10 +305,18 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-    // whole numbers (log2 units), minus infinity before the first key: m the
-    // largest reference of a block, l this lane's share of the sum times 2^-m;
-    // u the power of two of O, um the largest a block asked for
-    float m = -INFINITY, l = 0.f, u = -INFINITY, um = -INFINITY;
+    // m0: the maximum of the row's first block (log2 units). Alone it stays as
+    // it is: the largest weight of a row of few keys is 1 exactly. With more
+    // blocks to come it is rounded up to a multiple of 2^-16, to which whole
+    // numbers add without rounding. Whole numbers above m0, minus infinity
+    // before the first key: m the largest reference of a block, l this lane's
+    // share of the sum times 2^-m; u the power of two of O, um the largest a
+    // block asked for
+    float m0 = 0.f, m = -INFINITY, l = 0.f, u = -INFINITY, um = -INFINITY;
+    auto first = [&](float mb) {
+        const float c = b1 - b0 > KG && fabsf(mb) < 256.f ? ceilf(mb * 65536.f) * 0x1p-16f : mb;
+        if (m == -INFINITY && mb > -INFINITY) m0 = c;
+    };
     int last = 0;
     auto pow_of = [](float d) { return (int)fmaxf(d, -1000.f); };  // of a difference, which may be of infinities
 
@@ -354,7 +362,8 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int e = 0; e < 16; ++e) mb = fmaxf(mb, x[e]);
         mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-        const float rf = ceilf(mb), rz = mb == -INFINITY ? 0.f : rf;  // no key yet: every p is 0
+        if (__ballot(m == -INFINITY)) first(mb);
+        const float rf = ceilf(mb - m0), rz = mb == -INFINITY ? 0.f : rf + m0;  // no key yet: every p is 0
         // O takes this block's power of two (its largest p near 1, times V's),
         // at most 2^60 below the largest so far: what is smaller is below
         // every rounding of the row
@@ -439,7 +448,8 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int e = 0; e < 16; ++e) mb = fmaxf(mb, x[e]);
         mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-        const float rf = ceilf(mb), rz = mb == -INFINITY ? 0.f : rf, mn = fmaxf(m, rf);
+        if (__ballot(m == -INFINITY)) first(mb);
+        const float rf = ceilf(mb - m0), rz = mb == -INFINITY ? 0.f : rf + m0, mn = fmaxf(m, rf);
 #pragma unroll
         for (int e = 0; e < 16; ++e) lb += __builtin_amdgcn_exp2f(x[e] - rz);
         l = ldexpf(l, pow_of(m - mn)) + ldexpf(lb, pow_of(rf - mn));
@@ -453,8 +463,8 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
             for (int hh = 0; hh < 2; ++hh) {
                 const int key = b * kKB + 8 * (i >> 2) + 4 * hh + (i & 3);
                 if (key > pt) continue;
-                const float xs = hh == h ? own : other, rs = xs == -INFINITY ? 0.f : ceilf(xs);
-                const float ps = __builtin_amdgcn_exp2f(xs - rs);
+                const float xs = hh == h ? own : other, rs = xs == -INFINITY ? 0.f : ceilf(xs - m0);
+                const float ps = __builtin_amdgcn_exp2f(xs - (rs + m0));
                 const float* vp = vc + (row0 + key) * HD + 4 * h;  // read twice: the registers are full
                 float mv = 0.f;
 #pragma unroll 1
@@ -491,6 +501,7 @@ __global__ __launch_bounds__(64 * RT * KG) __attribute__((amdgpu_waves_per_eu(2)
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] = ldexpf(last ? -o[dt][e] : o[dt][e], un);
+    m += m0;
 
     // merge of the key groups, in group order
     if constexpr (KG > 1) {

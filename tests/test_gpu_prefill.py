@@ -604,3 +604,19 @@ def test_captured_attention_of_long_contexts(dev, H, KVH, hd, sp, nt):
     got, = _captured(dev, call, [do])
     want = do.read(np.float32)  # the last eager call's
     assert np.allclose(got, want, rtol=0, atol=8e-6 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("H,KVH,hd,nt", [(8, 1, 64, 200), (28, 4, 128, 40)])
+def test_prefill_attention_of_one_key(dev, H, KVH, hd, nt):
+    """The first token's weight is 1 exactly: its output is V to the split of
+    V alone, at most 2^-23 of a value and 2^-23 / sqrt(3) = 6.9e-8 over many."""
+    print(f"[gpu] pf attention of one key H={H} KVH={KVH} hd={hd} nt={nt}", flush=True)
+    rng = np.random.default_rng(hd)
+    num = den = 0.0
+    for _ in range(8):
+        qkv = rng.normal(0, 1, (nt, (H + 2 * KVH) * hd)).astype(np.float32)
+        K = np.zeros((KVH, nt, hd), np.float32)
+        got, _, v64 = _attn_case(dev, H, KVH, hd, 0, nt, nt, K, K.copy(), qkv)
+        v = np.repeat(v64[:, 0], H // KVH, 0)
+        num, den = num + ((got[0] - v) ** 2).sum(), den + (v ** 2).sum()
+    assert np.sqrt(num / den) <= 6.9e-8, np.sqrt(num / den)
